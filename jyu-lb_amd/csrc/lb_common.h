@@ -119,13 +119,16 @@ LBD bool resolve(const Dims& d, int& i, int& j, int& k, int& l, int& flip) {
 // A pointer known to be equal across the wave. Marking it keeps the compiler
 // from folding per-lane offsets into it early: the address of a load then
 // stays "scalar base + 32-bit lane offset" instead of one 64-bit vector
-// address per population held in registers until the store.
+// address per population held in registers until the store. The pointer is
+// named as one to global memory: made from an integer, it would be accessed
+// with flat instructions, which take no scalar base (a 64-bit vector address
+// per access) and count as LDS accesses too.
 template <class T>
 LBD T* uniform_ptr(T* p) {
     const uint64_t v = (uint64_t)p;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (T*)(((uint64_t)hi << 32) | lo);
+    return (T*)(__attribute__((address_space(1))) T*)(((uint64_t)hi << 32) | lo);
 }
 
 LBD void decompose(uint32_t c, int ny, int nzp, int& i, int& j, int& k) {
