@@ -255,23 +255,31 @@ LBD int64_t odd_loc(const StepParams& p, uint32_t m, int64_t e, int l, int i, in
 // tabulated per moving site (k_ladd_prep, 18 links) whenever the walls change;
 // the step kernel adds cff * sum with the sign of c_l's first component.
 template <int L>
-LBD double ladd_sum(const Dims& d, const double* vel, int64_t nq, int i, int j, int k) {
-    int yi = i - CI[L], yj = j - CJ[L], yk = k - CK[L], lp = L, fl = 0;
-    double u[3] = {0.0, 0.0, 0.0};
-    if (resolve(d, yi, yj, yk, lp, fl)) {
-        const int64_t y = ((int64_t)yi * d.ny + yj) * d.nzp + yk;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            double v = vel[(int64_t)a * nq + y];
-            u[a] = (fl >> a & 1) ? -v : v;
-        }
-    }
+LBD double ladd_combine(const double* u) {
     constexpr int c[3] = {CI[L], CJ[L], CK[L]};
     constexpr int a = c[0] != 0 ? 0 : (c[1] != 0 ? 1 : 2);
     constexpr int b = nnz(L) == 1 ? -1 : (a == 0 ? (c[1] != 0 ? 1 : 2) : 2);
     if constexpr (b < 0) return u[a];
     else if constexpr (c[a] == c[b]) return u[a] + u[b];
     else return u[a] - u[b];
+}
+// velocity of the solid site x - c_l
+LBD void ladd_wall(const Dims& d, const double* vel, int64_t nq, int i, int j, int k, int l, double* u) {
+    int yi = i - CI[l], yj = j - CJ[l], yk = k - CK[l], lp = l, fl = 0;
+    u[0] = u[1] = u[2] = 0.0;
+    if (!resolve(d, yi, yj, yk, lp, fl)) return;
+    const int64_t y = ((int64_t)yi * d.ny + yj) * d.nzp + yk;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        double v = vel[(int64_t)a * nq + y];
+        u[a] = (fl >> a & 1) ? -v : v;
+    }
+}
+template <int L>
+LBD double ladd_sum(const Dims& d, const double* vel, int64_t nq, int i, int j, int k) {
+    double u[3];
+    ladd_wall(d, vel, nq, i, j, k, L, u);
+    return ladd_combine<L>(u);
 }
 
 // table slot of link l (the rest population has none)
@@ -280,16 +288,20 @@ LBD constexpr int link_slot(int l) { return l < REST ? l : l - 1; }
 LBD constexpr bool ladd_plus(int l) { return (CI[l] != 0 ? CI[l] : CJ[l] != 0 ? CJ[l] : CK[l]) > 0; }
 
 template <class T>
-LBD void ladd_apply(const StepParams& p, uint32_t c, uint32_t m, T* f) {
-    const T den = (T)p.den[c];
+LBD T ladd_term(int l, T den, T u) {
     const T cff1 = T(2.0) * den * T(2.0 / 36.0) * T(3.0);
     const T cff2 = T(2.0) * den * T(1.0 / 36.0) * T(3.0);
+    const T term = (nnz(l) == 1 ? cff1 : cff2) * u;
+    return ladd_plus(l) ? term : -term;
+}
+template <class T>
+LBD void ladd_apply(const StepParams& p, uint32_t c, uint32_t m, T* f) {
+    const T den = (T)p.den[c];
     const double* U = p.ladd_u + (int64_t)p.mov_idx[c] * (Q - 1);
 #pragma unroll
     for (int l = 0; l < Q; ++l) {
         if (l == REST || !(m & (1u << l))) continue;
-        const T term = (nnz(l) == 1 ? cff1 : cff2) * (T)U[link_slot(l)];
-        f[l] = ladd_plus(l) ? f[l] + term : f[l] - term;
+        f[l] += ladd_term<T>(l, den, (T)U[link_slot(l)]);
     }
 }
 
@@ -306,6 +318,29 @@ struct AdjParams {
     const void* dseed;  // dissipation objective: the seeds of diss_site
 };
 
+// Two fused steps (k_pair): the tiling and the density Ladd's term reads.
+struct PairParams {
+    int TK, TJ;       // inner columns of a tile
+    int hk, hj;       // rim columns on each side: 1, or 0 where one tile spans wall to wall
+    uint32_t ntk, ntj;
+    int chunk;        // planes a workgroup sweeps
+    uint32_t total;   // workgroups: ntk * ntj * chunks
+    // Moving walls. mov: per cell, the moving links' slots (bits 0-17) and the
+    // site's wall velocity among wall[] (bits 18-19); rho_in / rho_out: per
+    // cell, the density of the step before and of the second step, read and
+    // written at moving sites
+    const uint32_t* mov;
+    double wall[4][3];
+    const double* rho_in;
+    double* rho_out;
+};
+constexpr int PAIR_WALLS = 4;
+constexpr int PAIR_MOVING = 1, PAIR_FULL = 2;
+// Columns of a tile, rim included, one per thread. FP64 arithmetic holds the
+// next plane's populations and a collision in 256 VGPRs (2 waves per SIMD);
+// FP32 arithmetic in 168 (3 waves per SIMD).
+constexpr int pair_threads(int prec) { return prec == LB_FP64 || prec == LB_FP32_STORAGE ? 512 : 768; }
+
 // Launchers of the per-precision kernels, defined in lb_kernels.h and
 // instantiated once per precision P in its own translation unit (lb_inst.hip,
 // built with LB_INST_P = P). The adjoint launchers exist for LB_FP64 and
@@ -313,6 +348,8 @@ struct AdjParams {
 template <int P> void launch_step_rlx(const StepParams& p, int rlx, bool odd, hipStream_t st);
 template <int P> void launch_adj_rlx(const StepParams& p, const AdjParams& x, int rlx, bool odd, hipStream_t st);
 template <int P> void launch_diss_rlx(const StepParams& p, int rlx, bool odd, hipStream_t st);
+template <int P>
+void launch_pair_rlx(const StepParams& p, const PairParams& q, int rlx, int feat, hipStream_t st);
 template <int P> void launch_init(const StepParams& p, hipStream_t st);
 template <int P> void launch_post_f(const StepParams& p, int next_odd, double* out, hipStream_t st);
 

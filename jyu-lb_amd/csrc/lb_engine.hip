@@ -648,11 +648,24 @@ struct lb_solver {
     uint32_t step_lds[2] = {0, 0};            // see StepParams::lds
     uint32_t step_tile = TILE;                // see StepParams::tile
     bool tune = false;                        // choose the step launch on the next long evolve (tune_step)
+    bool autotune = true;                     // LB_AUTOTUNE
     bool tune_xcd = true;                     // ... including the tile order (not pinned by the user)
     bool tune_verbose = false;
     uint32_t* mov_idx = nullptr;  // moving-site index per site (k_ladd_prep)
     double* ladd_u = nullptr;     // 18 Ladd velocity sums per moving site
-    size_t ladd_cap = 0;          // moving sites ladd_u has room for
+    size_t ladd_cap = 0;          // moving sites ladd_u and mov_cell have room for
+    uint32_t* mov_cell = nullptr;  // cell of each moving site
+    uint32_t nmov = 0;
+    uint32_t* mov_word = nullptr;  // paired steps with moving walls: PairParams::mov, and whether it holds
+    double* den2 = nullptr;        // (each site's walls share one of a few velocities); PairParams::rho_*
+    bool mov_pairs = false;
+    // paired steps of the dense layouts (k_pair): the request (LB_PAIR, as
+    // sp_pull), whether run_steps takes them, and their tiling
+    int pair = -1;
+    bool pair_on = false;
+    bool pair_tune = false;  // ... to be settled by timing both (tune_pair), with single steps until then
+    int pair_tile[3] = {0, 0, 0};  // LB_PAIR_TILE: inner columns along k and j, planes (0: pair_tiling chooses)
+    PairParams pq{};
     void* f = nullptr;
     uint32_t* mask = nullptr;
     uint8_t* wclass = nullptr;
@@ -748,8 +761,18 @@ static size_t tc_size(int prec) { return prec == LB_FP64 || prec == LB_FP32_STOR
 // sparse layout (whose kernels then read no cell index for them).
 static size_t rec_row(const lb_solver* s) { return s->sparse ? (size_t)s->nfp : (size_t)s->nq; }
 
+static void dfree(lb_solver* s, void** p, size_t n);
+
 static int dalloc(lb_solver* s, void** p, size_t n) {
     hipError_t e = hipMalloc(p, n);
+    if (e != hipSuccess && s->f2 && (s->pair_on || s->pair_tune) && !s->pull_active) {
+        // the paired steps' second array makes room: single steps in place
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(s->stream);
+        s->pair_on = s->pair_tune = false;
+        dfree(s, &s->f2, (size_t)s->fsize * ts_size(s->prec));
+        e = hipMalloc(p, n);
+    }
     if (e != hipSuccess) {
         *p = nullptr;
         return fail(LB_ENOMEM, "hipMalloc(%zu bytes) failed: %s", n, hipGetErrorString(e));
@@ -957,7 +980,7 @@ LBD void ladd_sums(const Dims& d, const double* vel, int64_t nq, int i, int j, i
 }
 
 __global__ void k_ladd_prep(const uint32_t* mask, const double* vel, Dims d, uint32_t nq, uint32_t* mov_idx,
-                            double* ladd_u, unsigned int* counter) {
+                            double* ladd_u, uint32_t* mov_cell, unsigned int* counter) {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nq) return;  // whole waves only: nq % 64 == 0
     const uint32_t m = mask[c];
@@ -971,6 +994,7 @@ __global__ void k_ladd_prep(const uint32_t* mask, const double* vel, Dims d, uin
     if (!mv) return;
     const uint32_t q = base + __popcll(b & ((1ull << lane) - 1ull));
     mov_idx[c] = q;
+    mov_cell[q] = c;
     int i, j, k;
     decompose(c, d.ny, d.nzp, i, j, k);
     double* out = ladd_u + (int64_t)q * (Q - 1);
@@ -979,6 +1003,61 @@ __global__ void k_ladd_prep(const uint32_t* mask, const double* vel, Dims d, uin
 #pragma unroll
     for (int l = 0; l < Q; ++l)
         if (l != REST) out[link_slot(l)] = tmp[l];
+}
+
+// The paired steps' form of the moving sites (PairParams::mov): site q's
+// moving links, and its wall velocity among the n in walls. *first becomes the
+// lowest q whose velocity is not among them, or 0 where one site's walls
+// differ (*split).
+struct Walls {
+    double v[PAIR_WALLS][3];
+    int n;
+};
+LBD bool same_bits(const double* a, const double* b) {
+    for (int x = 0; x < 3; ++x)
+        if (__double_as_longlong(a[x]) != __double_as_longlong(b[x])) return false;
+    return true;
+}
+// wall velocity of moving site c, its moving links, and whether they agree
+LBD bool site_wall(const uint32_t* mask, const double* vel, const Dims& d, uint32_t nq, uint32_t c, double* v,
+                   uint32_t& links) {
+    int i, j, k;
+    decompose(c, d.ny, d.nzp, i, j, k);
+    links = 0;
+    bool one = true;
+    for (int l = 0; l < Q; ++l) {
+        if (l == REST || !(mask[c] & (1u << l))) continue;
+        double u[3];
+        ladd_wall(d, vel, nq, i, j, k, l, u);
+        if (u[0] == 0.0 && u[1] == 0.0 && u[2] == 0.0) continue;
+        if (!links)
+            for (int a = 0; a < 3; ++a) v[a] = u[a];
+        else if (!same_bits(u, v)) one = false;
+        links |= 1u << link_slot(l);
+    }
+    return one;
+}
+__global__ void k_pair_walls(const uint32_t* mask, const double* vel, Dims d, uint32_t nq, const uint32_t* cell,
+                             uint32_t n, Walls walls, uint32_t* word, unsigned int* first, unsigned int* split) {
+    const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    double v[3] = {0.0, 0.0, 0.0};
+    uint32_t links;
+    if (!site_wall(mask, vel, d, nq, cell[q], v, links)) atomicOr(split, 1u);
+    int e = 0;
+    while (e < walls.n && !same_bits(v, walls.v[e])) ++e;
+    if (e == walls.n) atomicMin(first, q);
+    else word[cell[q]] = links | (uint32_t)e << 18;
+}
+__global__ void k_wall_of(const uint32_t* mask, const double* vel, Dims d, uint32_t nq, const uint32_t* cell,
+                          const unsigned int* q, double* v) {
+    uint32_t links;
+    site_wall(mask, vel, d, nq, cell[*q], v, links);
+}
+// densities of the moving sites from one array to the other
+__global__ void k_rho_copy(const uint32_t* cell, uint32_t n, const double* from, double* to) {
+    const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < n) to[cell[q]] = from[cell[q]];
 }
 
 // sparse layout set-up: fluid sites per wave of 64 sites
@@ -1102,6 +1181,43 @@ __global__ __launch_bounds__(64) void k_sparse_pack(const uint32_t* tab, uint32_
     ((uint8_t*)(tabc + (size_t)SP_WORDS * nfp))[n] = (uint8_t)word[SP_WORDS];
 }
 
+// Whether the paired steps can take this lattice's moving walls (mov_pairs),
+// and their form of them: every site's moving walls share one velocity, and
+// there are at most PAIR_WALLS of those (a lid, two sliding plates). Each
+// round finds one more velocity. Other walls keep single steps, which read 18
+// sums per site: in the paired steps those loads wait behind the next plane's
+// (256^3 cavity, FP64: 0.713 ms per step with the sums loaded, 0.648 so; 48^3
+// 0.0128 and 0.0102).
+static int pair_walls(lb_solver* s) {
+    s->mov_pairs = false;
+    int rc;
+    if (!s->mov_word && (rc = dalloc(s, (void**)&s->mov_word, (size_t)s->nq * 4))) return rc;
+    if (!s->den2 && (rc = dalloc(s, (void**)&s->den2, (size_t)s->nq * 8))) return rc;
+    Walls walls;
+    memset(&walls, 0, sizeof(walls));
+    unsigned int* first = (unsigned int*)s->red;  // first, split; the velocity after them
+    double* v = s->red + 1;
+    for (;; ++walls.n) {
+        const unsigned int init[2] = {~0u, 0u};
+        unsigned int got[2];
+        HIPCHK(hipMemcpyAsync(first, init, sizeof(init), hipMemcpyHostToDevice, s->stream));
+        k_pair_walls<<<blocks_for(s->nmov, 256), 256, 0, s->stream>>>(s->mask, s->vel, s->d, s->nq, s->mov_cell, s->nmov,
+                                                                      walls, s->mov_word, first, first + 1);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(got, first, sizeof(got), hipMemcpyDeviceToHost, s->stream));
+        HIPCHK(hipStreamSynchronize(s->stream));
+        if (got[1] || (got[0] != ~0u && walls.n == PAIR_WALLS)) return LB_OK;
+        if (got[0] == ~0u) break;
+        k_wall_of<<<1, 1, 0, s->stream>>>(s->mask, s->vel, s->d, s->nq, s->mov_cell, first, v);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(walls.v[walls.n], v, 24, hipMemcpyDeviceToHost, s->stream));
+        HIPCHK(hipStreamSynchronize(s->stream));
+    }
+    memcpy(s->pq.wall, walls.v, sizeof(walls.v));
+    s->mov_pairs = true;
+    return LB_OK;
+}
+
 static int count_mask(lb_solver* s, int64_t* nfluid, int64_t* nmoving) {
     unsigned long long* d = (unsigned long long*)s->red;
     HIPCHK(hipMemsetAsync(d, 0, 32, s->stream));
@@ -1137,6 +1253,7 @@ static int count_mask(lb_solver* s, int64_t* nfluid, int64_t* nmoving) {
         HIPCHK(hipStreamSynchronize(s->stream));
     }
     const size_t nmov = (size_t)*nmoving;
+    s->nmov = (uint32_t)nmov;
     if (nmov > 0) {
         int rc;
         if (!s->mov_idx && (rc = dalloc(s, (void**)&s->mov_idx, (size_t)s->nq * 4))) return rc;
@@ -1145,16 +1262,21 @@ static int count_mask(lb_solver* s, int64_t* nfluid, int64_t* nmoving) {
                 HIPCHK(hipFree(s->ladd_u));
                 s->bytes -= s->ladd_cap * (Q - 1) * 8;
                 s->ladd_u = nullptr;
+                dfree(s, (void**)&s->mov_cell, s->ladd_cap * 4);
+                s->ladd_cap = 0;
             }
-            if ((rc = dalloc(s, (void**)&s->ladd_u, nmov * (Q - 1) * 8))) return rc;
+            if ((rc = dalloc(s, (void**)&s->ladd_u, nmov * (Q - 1) * 8)) ||
+                (rc = dalloc(s, (void**)&s->mov_cell, nmov * 4)))
+                return rc;
             s->ladd_cap = nmov;
         }
         unsigned int* cnt = (unsigned int*)s->red;
         HIPCHK(hipMemsetAsync(cnt, 0, 4, s->stream));
         k_ladd_prep<<<blocks_for(s->nq, 256), 256, 0, s->stream>>>(s->mask, s->vel, s->d, s->nq, s->mov_idx,
-                                                                  s->ladd_u, cnt);
+                                                                  s->ladd_u, s->mov_cell, cnt);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s->stream));
+        if (s->finalized && (s->pair_on || s->pair_tune) && (rc = pair_walls(s))) return rc;  // else at lb_finalize's end
     }
     return LB_OK;
 }
@@ -1184,6 +1306,18 @@ static void launch_any_step(const lb_solver* s, const StepParams& ps, bool odd) 
     case LB_FP32_SHIFTED: launch_step_rlx<LB_FP32_SHIFTED>(p, s->cfg.rlx_scheme, odd, s->stream); break;
     case LB_FP32_STORAGE: launch_step_rlx<LB_FP32_STORAGE>(p, s->cfg.rlx_scheme, odd, s->stream); break;
     default: launch_step_rlx<LB_FP16_STORAGE>(p, s->cfg.rlx_scheme, odd, s->stream); break;
+    }
+}
+
+static void launch_any_pair(const lb_solver* s, const StepParams& p, const PairParams& q) {
+    const bool sym = s->d.bc[2] == SYMMETRIC || s->d.bc[3] == SYMMETRIC || s->d.bc[4] == SYMMETRIC ||
+                     s->d.bc[5] == SYMMETRIC;
+    const int feat = (s->nzh || sym || p.acc ? PAIR_FULL : 0) | (s->moving ? PAIR_MOVING : 0);
+    switch (s->prec) {
+    case LB_FP64: launch_pair_rlx<LB_FP64>(p, q, s->cfg.rlx_scheme, feat, s->stream); break;
+    case LB_FP32_SHIFTED: launch_pair_rlx<LB_FP32_SHIFTED>(p, q, s->cfg.rlx_scheme, feat, s->stream); break;
+    case LB_FP32_STORAGE: launch_pair_rlx<LB_FP32_STORAGE>(p, q, s->cfg.rlx_scheme, feat, s->stream); break;
+    default: launch_pair_rlx<LB_FP16_STORAGE>(p, q, s->cfg.rlx_scheme, feat, s->stream); break;
     }
 }
 
@@ -1249,6 +1383,13 @@ static void layout_defaults(lb_solver* s, int layout) {
     s->sp_pull = -1;  // decided by sp_pull_on at lb_finalize
     if (const char* env = getenv("LB_SP_PULL")) s->sp_pull = strtol(env, nullptr, 10) != 0 ? 1 : 0;
     s->adj_pull = -1;
+    s->pair = -1;
+    if (const char* env = getenv("LB_PAIR")) s->pair = strtol(env, nullptr, 10) != 0 ? 1 : 0;
+    if (const char* env = getenv("LB_PAIR_TILE")) {
+        int v[3];
+        if (sscanf(env, "%d,%d,%d", v, v + 1, v + 2) == 3 && v[0] > 0 && v[1] > 0 && v[2] > 0)
+            for (int a = 0; a < 3; ++a) s->pair_tile[a] = v[a];
+    }
     if (const char* env = getenv("LB_ADJ_PULL")) s->adj_pull = strtol(env, nullptr, 10) != 0 ? 1 : 0;
     if (const char* env = getenv("LB_XCD_CHUNK")) {
         s->xcd_chunk = (uint32_t)strtoul(env, nullptr, 10);
@@ -1282,6 +1423,93 @@ static void layout_defaults(lb_solver* s, int layout) {
         const unsigned long t = strtoul(env, nullptr, 10);
         if (t >= 64 && t <= (unsigned long)STEP_TILE_MAX && t % 64 == 0) s->step_tile = (uint32_t)t;
     }
+}
+
+// Whether a dense layout steps in pairs (k_pair) where a call has two steps
+// left: not with a symmetric x face (the sweep along i does not mirror), nor
+// where three planes of populations exceed the kernel's 32-bit offsets, nor
+// where LB_SP_PULL asks for single steps of one kind. rs and ps are set.
+static bool pair_wanted(const lb_solver* s) {
+    if (s->sparse || s->sp_pull >= 0 || s->pair == 0) return false;
+    if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
+    const uint64_t ts = ts_size(s->prec);
+    return 3 * (uint64_t)s->d.ny * (uint64_t)s->rs * ts + Q * (uint64_t)s->ps * ts < (1ull << 32);
+}
+
+// The tiling of the paired steps: inner columns along k and j, planes per
+// workgroup. A workgroup runs two iterations more than it stores planes, and
+// about one more to start; a CU holds one workgroup at a time, so a launch
+// takes ceil(workgroups / CUs) of them. An iteration (us) has a part that no
+// column shortens (two barriers, LDS, a collision's chain) and one by the
+// column, which the lines its row reads raise: 34 doubles span 3.4 lines of
+// 128 bytes on average, 66 span 5.4. Measured with every tiling forced in
+// turn: 256^3 FP64 0.593 ms per step at 32x13x32 (predicted best), 0.642 at
+// 16x26x32, 0.681 at 64x5x32; 512x128x128 FP32 0.191 at 64x8x64 (predicted
+// best), 0.204 at 32x16x64; 48^3 FP64 0.0085 at 24x6x3 (predicted best),
+// 0.0096 at 48x8x2.
+static void pair_tiling(lb_solver* s) {
+    const Dims& d = s->d;
+    const int NT = pair_threads(s->prec);
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    const bool perk = d.bc[4] == PERIODIC, perj = d.bc[2] == PERIODIC;
+    const double per_line = 128.0 / (double)ts_size(s->prec);
+    PairParams best{};
+    double tbest = 0.0;
+    auto consider = [&](int TK, int TJ, int chunk) {
+        PairParams q{};
+        q.TK = TK;
+        q.TJ = TJ;
+        q.ntk = (uint32_t)((d.nz + TK - 1) / TK);
+        q.ntj = (uint32_t)((d.ny + TJ - 1) / TJ);
+        q.hk = q.ntk > 1 || perk;
+        q.hj = q.ntj > 1 || perj;
+        q.chunk = chunk;
+        const int EK = TK + 2 * q.hk, cols = EK * (TJ + 2 * q.hj);
+        if (cols > NT) return;
+        const uint64_t total = (uint64_t)q.ntk * q.ntj * (uint64_t)((d.nx + chunk - 1) / chunk);
+        if (total > (1u << 30)) return;
+        q.total = (uint32_t)total;
+        const double lines = 1.0 + 1.3 * per_line / EK;  // lines read over lines needed
+        const double iter = 1.3 + 4.6 * cols / NT * (0.5 + 0.5 * lines / 1.6);
+        const double t = (double)((total + cus - 1) / cus) * (chunk + 3) * iter;
+        if (!best.total || t < tbest) {
+            best = q;
+            tbest = t;
+        }
+    };
+    // the sizes that split n into fewer equal parts than the next smaller one
+    auto sizes = [](int n, int most, auto f) {
+        for (int parts = (n + most - 1) / most;;) {
+            const int size = (n + parts - 1) / parts;
+            f(size);
+            if (size == 1) break;
+            parts = (n + size - 2) / (size - 1);
+        }
+    };
+    auto all_of = [&](int TK) {
+        const bool rim = (d.nz + TK - 1) / TK > 1 || perk;
+        sizes(d.ny, std::min(d.ny, NT / (TK + 2 * rim)),
+              [&](int TJ) { sizes(d.nx, d.nx, [&](int chunk) { consider(TK, TJ, chunk); }); });
+    };
+    if (s->pair_tile[0])
+        consider(std::min(s->pair_tile[0], d.nz), std::min(s->pair_tile[1], d.ny), std::min(s->pair_tile[2], d.nx));
+    if (!best.total) {
+        for (int ntk = 1; ntk <= d.nz; ++ntk) {
+            const int TK = (d.nz + ntk - 1) / ntk, TK8 = (TK + 7) / 8 * 8;
+            if (TK > NT / 3) continue;
+            if (ntk > 1 && TK < 20) break;
+            all_of(ntk > 1 ? TK8 : TK);  // tiles start on half a line at least: unaligned ones (37x11x86) ran 256^3 FP64 at 0.886
+        }
+    }
+    memcpy(best.wall, s->pq.wall, sizeof(best.wall));
+    s->pq = best;
+    if (!best.total) s->pair_on = false;
+    if (s->tune_verbose && s->pair_on)
+        fprintf(stderr, "[jyulb] paired steps: tiles of %d x %d columns, %d planes, %u workgroups\n", best.TK, best.TJ,
+                best.chunk, best.total);
 }
 
 // Strides and population array of a layout: row-interleaved f[i][j][l][k]
@@ -1318,12 +1546,13 @@ static int layout_arrays(lb_solver* s, int layout) {
         if (s->f2) HIPCHK(hipMemset(s->f2, 0, fb));
         s->pull_active = s->f2 && s->sp_pull == 1;
     }
+    s->pair_on = pair_wanted(s);
     return LB_OK;
 }
 
 // The second array of a dense pull-step candidate that was not chosen.
 static void drop_pull_candidate(lb_solver* s) {
-    if (s->f2 && !s->pull_active) dfree(s, &s->f2, (size_t)s->fsize * ts_size(s->prec));
+    if (s->f2 && !s->pull_active && !s->pair_on && !s->pair_tune) dfree(s, &s->f2, (size_t)s->fsize * ts_size(s->prec));
 }
 
 int lb_create(const lb_config* cfg, lb_solver** out) {
@@ -1355,7 +1584,8 @@ int lb_create(const lb_config* cfg, lb_solver** out) {
         uint64_t min_cells = TUNE_MIN_CELLS;
         if (const char* env = getenv("LB_AUTOTUNE_MIN_CELLS")) min_cells = strtoull(env, nullptr, 10);
         const char* at = getenv("LB_AUTOTUNE");
-        s->tune = (!at || strtol(at, nullptr, 10) != 0) && !getenv("LB_STEP_TILE") && !getenv("LB_STEP_LDS_EVEN") &&
+        s->autotune = !at || strtol(at, nullptr, 10) != 0;
+        s->tune = s->autotune && !getenv("LB_STEP_TILE") && !getenv("LB_STEP_LDS_EVEN") &&
                   !getenv("LB_STEP_LDS_ODD") && (uint64_t)s->nq >= min_cells;
         const char* vb = getenv("LB_AUTOTUNE_VERBOSE");
         s->tune_verbose = vb && strtol(vb, nullptr, 10) != 0;
@@ -1424,7 +1654,7 @@ int lb_destroy(lb_solver* s) {
     void* ptrs[] = {s->f,     s->mask, s->wclass, s->special, s->phase, s->den,  s->vel,  s->acc,
                     s->stage, s->part, s->red,    s->uprev,   s->ckpt,  s->lam,  s->lam2, s->rec,  s->gacc, s->gface,
                     s->snap,  s->snap_dv, s->mov_idx, s->ladd_u, s->cidx, s->site, s->tab,
-                    s->tabc, s->tabw, s->f2, s->prev, s->dseed, s->st_phase, s->st_den, s->st_vel, s->st_acc};
+                    s->mov_cell, s->mov_word, s->den2, s->tabc, s->tabw, s->f2, s->prev, s->dseed, s->st_phase, s->st_den, s->st_vel, s->st_acc};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (int f = 0; f < 6; ++f) {
@@ -1623,6 +1853,21 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
         if ((rc = layout_arrays(s, layout))) return rc;
     }
     if (s->sparse && (rc = build_sparse(s))) return rc;
+    if (s->pair_tune) s->pair_on = true;  // finalized again
+    if (s->pair_on) pair_tiling(s);
+    if (s->pair_on && s->moving && (rc = pair_walls(s))) return rc;
+    if (s->pair_on) {
+        // Pairs are faster where walls stand still and values have 4 bytes or
+        // more (ms per step, single / paired: 256^3 channel FP64 0.894 /
+        // 0.593, FP32 0.451 / 0.323; 160^3 FP32 0.121 / 0.119; 48^3 FP64
+        // 0.0215 / 0.0085). With moving walls or FP16 storage, where the
+        // collisions bind, it depends: cavities 256^3 FP64 0.928 / 0.648, FP16
+        // 0.284 / 0.389, 160^3 FP32 0.118 / 0.132, 64^3 FP64 0.0164 / 0.0171,
+        // 48^3 FP64 0.0128 / 0.0102; 64^3 channel FP16 0.0184 / 0.0112.
+        s->pair_tune = s->pair < 0 && s->autotune && (s->moving || s->prec == LB_FP16_STORAGE);
+        if (s->pair_tune) s->pair_on = false;
+        else s->tune = false;  // few single steps are left to tune
+    }
     if (s->prec == LB_FP16_STORAGE && s->f16_auto) {
         k_maxdev<<<256, 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->nq, s->rho0, s->part);
         HIPCHK(hipGetLastError());
@@ -1753,19 +1998,79 @@ static void one_step(lb_solver* s, StepParams& p, int& odd) {
     }
 }
 
+static bool capturing(const lb_solver* s) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s->stream, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return capture != hipStreamCaptureStatusNone;
+}
+
+// Whether this call's steps may be paired: the second population array is
+// there (the first such call allocates it; without the memory, steps stay
+// single) and the stream is not being captured, as a graph replays with the
+// arrays it was captured with, while pairs swap them.
+static bool pairs_ready(lb_solver* s) {
+    if (!s->pair_on || (s->moving && !s->mov_pairs)) return false;
+    if (capturing(s)) return false;
+    if (s->f2) return true;
+    const size_t fb = (size_t)s->fsize * ts_size(s->prec);
+    dalloc_optional(s, &s->f2, fb);
+    if (s->f2 && s->prec == LB_FP16_STORAGE)  // the FP16 guard reads more than the fluid sites
+        k_fill<uint64_t><<<(unsigned)((fb / 8 + 255) / 256), 256, 0, s->stream>>>((uint64_t*)s->f2, fb / 8, 0);
+    s->pair_on = s->f2 != nullptr;
+    return s->pair_on;
+}
+
+static void swap_rho(PairParams& q) {
+    const double* in = q.rho_out;
+    q.rho_out = const_cast<double*>(q.rho_in);
+    q.rho_in = in;
+}
+
 static int run_steps(lb_solver* s, uint32_t n, bool store_last) {
     StepParams p = params(s);
-    for (uint32_t t = 0; t < n; ++t) {
+    PairParams q = s->pq;
+    // moving walls: the moving sites' last densities are in den or in den2
+    q.mov = s->mov_word;
+    q.rho_in = s->den;
+    q.rho_out = s->den2;
+    auto move_rho = [&] {  // to the other array
+        k_rho_copy<<<blocks_for(s->nmov, 256), 256, 0, s->stream>>>(s->mov_cell, s->nmov, q.rho_in, q.rho_out);
+        swap_rho(q);
+    };
+    const bool pairs = n >= 2 && pairs_ready(s);
+    for (uint32_t t = 0; t < n;) {
         if (s->prec == LB_FP16_STORAGE && s->f16_since >= s->f16_check) {
             int rc = fp16_guard(s);
             if (rc) return rc;
             p = params(s);
         }
-        p.store_dv = (store_last && t + 1 == n) ? 1 : 0;
-        one_step(s, p, s->next_odd);
-        s->steps++;
-        s->f16_since++;
+        // two steps at once from the state an even step leaves; a pair does
+        // not reach past the next FP16 check
+        const bool pair = pairs && s->next_odd && n - t >= 2 &&
+                          (s->prec != LB_FP16_STORAGE || s->f16_since + 2 <= s->f16_check);
+        const uint32_t len = pair ? 2u : 1u;
+        p.store_dv = (store_last && t + len == n) ? 1 : 0;
+        if (pair) {
+            // the last pair stores den, which its tiles' rims must not read
+            if (s->moving && p.store_dv && q.rho_in == s->den) move_rho();
+            p.f2 = s->f2;
+            launch_any_pair(s, p, q);
+            std::swap(s->f, s->f2);
+            p.f = s->f;
+            p.f2 = nullptr;
+            if (s->moving) swap_rho(q);
+        } else {
+            if (s->moving && q.rho_in != s->den) move_rho();
+            one_step(s, p, s->next_odd);
+        }
+        s->steps += len;
+        s->f16_since += len;
+        t += len;
     }
+    if (s->moving && q.rho_in != s->den) move_rho();
     return LB_OK;
 }
 
@@ -1926,6 +2231,37 @@ static int tune_step(lb_solver* s) {
     return tune_pull(s);
 }
 
+// Single or paired steps, by timing the call's own: PAIR_TUNE single steps and
+// as many paired ones, each after two that are not counted. The results are
+// the same either way.
+constexpr int PAIR_TUNE = 8, PAIR_TUNE_STEPS = 2 * (PAIR_TUNE + 2) + 1;
+static int tune_pair(lb_solver* s) {
+    hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    bool ok = true;
+    for (hipEvent_t& e : ev) ok = ok && hipEventCreate(&e) == hipSuccess;
+    int rc = LB_OK;
+    float ms[2] = {0.0f, 0.0f};
+    if (ok && !s->next_odd) rc = run_steps(s, 1, false);  // pairs start from the state an even step leaves
+    for (int k = 0; ok && !rc && k < 2; ++k) {
+        s->pair_on = k == 1;
+        if ((rc = run_steps(s, 2, false))) break;
+        ok = hipEventRecord(ev[2 * k], s->stream) == hipSuccess;
+        if ((rc = run_steps(s, PAIR_TUNE, false))) break;
+        ok = ok && hipEventRecord(ev[2 * k + 1], s->stream) == hipSuccess;
+    }
+    ok = ok && !rc && hipEventSynchronize(ev[3]) == hipSuccess;
+    for (int k = 0; ok && k < 2; ++k) ok = hipEventElapsedTime(&ms[k], ev[2 * k], ev[2 * k + 1]) == hipSuccess;
+    for (hipEvent_t e : ev)
+        if (e) (void)hipEventDestroy(e);
+    s->pair_tune = false;
+    s->pair_on = ok && ms[1] < ms[0];
+    if (s->tune_verbose)
+        fprintf(stderr, "[jyulb] single steps %.4f ms, paired steps %.4f ms per step\n", ms[0] / PAIR_TUNE,
+                ms[1] / PAIR_TUNE);
+    drop_pull_candidate(s);
+    return rc;
+}
+
 // The state before a call's last step, kept for the reference's f2: after
 // evolve the reference's f2 holds the post-collision populations of the
 // step before the last one (its two arrays are swapped every step,
@@ -1967,6 +2303,11 @@ static int evolve_steps(lb_solver* s, uint32_t steps) {
             if ((rc = tune_step(s))) return rc;
             steps -= (uint32_t)(s->steps - before);
         }
+    }
+    if (s->pair_tune && !s->tune && steps > (uint32_t)PAIR_TUNE_STEPS && !capturing(s)) {
+        const uint64_t before = s->steps;
+        if ((rc = tune_pair(s))) return rc;
+        steps -= (uint32_t)(s->steps - before);
     }
     if (s->keep_prev) {
         if ((rc = run_steps(s, steps - 1, false)) || (rc = capture_prev(s)) || (rc = run_steps(s, 1, true)))

@@ -10,6 +10,7 @@
 namespace lb {
 
 template void launch_step_rlx<LB_INST_P>(const StepParams&, int, bool, hipStream_t);
+template void launch_pair_rlx<LB_INST_P>(const StepParams&, const PairParams&, int, int, hipStream_t);
 template void launch_init<LB_INST_P>(const StepParams&, hipStream_t);
 template void launch_post_f<LB_INST_P>(const StepParams&, int, double*, hipStream_t);
 #if LB_INST_P == LB_FP64 || LB_INST_P == LB_FP32_SHIFTED

@@ -537,6 +537,10 @@ __global__ __launch_bounds__(STEP_TILE_MAX) void k_diss_sp(StepParams p) {
     step_sparse<P, RLX, ODD, FULL, true>(p, n);
 }
 
+}  // namespace lb
+#include "lb_pair.h"
+namespace lb {
+
 // ---------------------------------------------------------------------------
 // adjoint step
 // ---------------------------------------------------------------------------

@@ -63,27 +63,11 @@ LBD void moments_h(const T* f, T* h) {
 
 // Kinetic projection P(h): h_to_f (D3Q19.pyx:460-527) when ADD is false,
 // add_h_to_f (D3Q19.pyx:532-599) when true. DIV corrects the products with
-// the rounded reciprocals of 72 and 3 to the quotients.
-template <class T, bool ADD, bool DIV = false>
+// the rounded reciprocals of 72 and 3 to the quotients. LEAN keeps the
+// compiler from holding all 19 terms at once: each plane's four go to f before
+// the next are formed (in a kernel that is short of registers).
+template <class T, bool ADD, bool DIV = false, bool LEAN = false>
 LBD void project(const T* h, T* f) {
-    T e_xy = T(2) * h[0] + T(6) * h[4] + T(6) * h[7] - T(3) * h[9];
-    T e_1x_1y = e_xy + T(18) * h[5];
-    T o_1x_1y = T(-6) * h[1] - T(6) * h[2];
-    T e_1x_y1 = e_xy - T(18) * h[5];
-    T o_1x_y1 = T(-6) * h[1] + T(6) * h[2];
-    T e_xz = T(2) * h[0] + T(6) * h[4] - T(3) * h[7] + T(6) * h[9];
-    T e_1x_1z = e_xz + T(18) * h[6];
-    T o_1x_1z = T(-6) * h[1] - T(6) * h[3];
-    T e_1x_z1 = e_xz - T(18) * h[6];
-    T o_1x_z1 = T(-6) * h[1] + T(6) * h[3];
-    T e_yz = T(2) * h[0] - T(3) * h[4] + T(6) * h[7] + T(6) * h[9];
-    T e_1y_1z = e_yz + T(18) * h[8];
-    T o_1y_1z = T(-6) * h[2] - T(6) * h[3];
-    T e_1y_z1 = e_yz - T(18) * h[8];
-    T o_1y_z1 = T(-6) * h[2] + T(6) * h[3];
-    T e_1x = T(4) * h[0] + T(12) * h[4] - T(6) * h[7] - T(6) * h[9];
-    T e_1y = T(4) * h[0] - T(6) * h[4] + T(12) * h[7] - T(6) * h[9];
-    T e_1z = T(4) * h[0] - T(6) * h[4] - T(6) * h[7] + T(12) * h[9];
     // In FP32 the rounded 1/72 and 1/3 are 7.5e-9 and 3e-8 too large, a bias
     // that every step applies to every moment. DIV removes it: the product
     // with the rounded reciprocal is corrected by its remainder v - q d, which
@@ -101,27 +85,57 @@ LBD void project(const T* h, T* f) {
     };
     auto c72 = [&](T v) { return quo(v, T(72.0)); };
     T p[19];
-    p[0] = c72(e_1x_1y + o_1x_1y);
-    p[18] = c72(e_1x_1y - o_1x_1y);
-    p[1] = c72(e_1x_1z + o_1x_1z);
-    p[17] = c72(e_1x_1z - o_1x_1z);
-    p[2] = c72(e_1x - T(12) * h[1]);
-    p[16] = c72(e_1x + T(12) * h[1]);
-    p[3] = c72(e_1x_z1 + o_1x_z1);
-    p[15] = c72(e_1x_z1 - o_1x_z1);
-    p[4] = c72(e_1x_y1 + o_1x_y1);
-    p[14] = c72(e_1x_y1 - o_1x_y1);
-    p[5] = c72(e_1y_1z + o_1y_1z);
-    p[13] = c72(e_1y_1z - o_1y_1z);
-    p[6] = c72(e_1y - T(12) * h[2]);
-    p[12] = c72(e_1y + T(12) * h[2]);
-    p[7] = c72(e_1y_z1 + o_1y_z1);
-    p[11] = c72(e_1y_z1 - o_1y_z1);
-    p[8] = c72(e_1z - T(12) * h[3]);
-    p[10] = c72(e_1z + T(12) * h[3]);
-    p[9] = quo(h[0], T(3.0)) - T(0.5) * (h[4] + h[7] + h[9]);
+    auto put = [&](int l, T v) {
+        if constexpr (LEAN) f[l] = ADD ? f[l] + v : v;
+        else p[l] = v;
+    };
+    auto next = [] {
+        if constexpr (LEAN) __builtin_amdgcn_sched_barrier(0);
+    };
+    T e_xy = T(2) * h[0] + T(6) * h[4] + T(6) * h[7] - T(3) * h[9];
+    T e_1x_1y = e_xy + T(18) * h[5];
+    T o_1x_1y = T(-6) * h[1] - T(6) * h[2];
+    T e_1x_y1 = e_xy - T(18) * h[5];
+    T o_1x_y1 = T(-6) * h[1] + T(6) * h[2];
+    put(0, c72(e_1x_1y + o_1x_1y));
+    put(18, c72(e_1x_1y - o_1x_1y));
+    put(4, c72(e_1x_y1 + o_1x_y1));
+    put(14, c72(e_1x_y1 - o_1x_y1));
+    next();
+    T e_xz = T(2) * h[0] + T(6) * h[4] - T(3) * h[7] + T(6) * h[9];
+    T e_1x_1z = e_xz + T(18) * h[6];
+    T o_1x_1z = T(-6) * h[1] - T(6) * h[3];
+    T e_1x_z1 = e_xz - T(18) * h[6];
+    T o_1x_z1 = T(-6) * h[1] + T(6) * h[3];
+    put(1, c72(e_1x_1z + o_1x_1z));
+    put(17, c72(e_1x_1z - o_1x_1z));
+    put(3, c72(e_1x_z1 + o_1x_z1));
+    put(15, c72(e_1x_z1 - o_1x_z1));
+    next();
+    T e_yz = T(2) * h[0] - T(3) * h[4] + T(6) * h[7] + T(6) * h[9];
+    T e_1y_1z = e_yz + T(18) * h[8];
+    T o_1y_1z = T(-6) * h[2] - T(6) * h[3];
+    T e_1y_z1 = e_yz - T(18) * h[8];
+    T o_1y_z1 = T(-6) * h[2] + T(6) * h[3];
+    put(5, c72(e_1y_1z + o_1y_1z));
+    put(13, c72(e_1y_1z - o_1y_1z));
+    put(7, c72(e_1y_z1 + o_1y_z1));
+    put(11, c72(e_1y_z1 - o_1y_z1));
+    next();
+    T e_1x = T(4) * h[0] + T(12) * h[4] - T(6) * h[7] - T(6) * h[9];
+    T e_1y = T(4) * h[0] - T(6) * h[4] + T(12) * h[7] - T(6) * h[9];
+    T e_1z = T(4) * h[0] - T(6) * h[4] - T(6) * h[7] + T(12) * h[9];
+    put(2, c72(e_1x - T(12) * h[1]));
+    put(16, c72(e_1x + T(12) * h[1]));
+    put(6, c72(e_1y - T(12) * h[2]));
+    put(12, c72(e_1y + T(12) * h[2]));
+    put(8, c72(e_1z - T(12) * h[3]));
+    put(10, c72(e_1z + T(12) * h[3]));
+    put(9, quo(h[0], T(3.0)) - T(0.5) * (h[4] + h[7] + h[9]));
+    if constexpr (!LEAN) {
 #pragma unroll
-    for (int l = 0; l < Q; ++l) f[l] = ADD ? f[l] + p[l] : p[l];
+        for (int l = 0; l < Q; ++l) f[l] = ADD ? f[l] + p[l] : p[l];
+    }
 }
 
 // den_vel_to_heq, D3Q19.pyx:604-630
@@ -158,7 +172,7 @@ LBD void forcing(T* h, const T* acc, T den, T jx, T jy, T jz, T c1, T c2) {
 // the half-force shifted velocity, ds the density as the populations hold it
 // (den, or den - rho0 when SH: the caller can add rho0 back in FP64, where
 // den itself carries only the compute type's precision near rho0).
-template <class T, bool SH, bool DIV = false>
+template <class T, bool SH, bool DIV = false, bool LEAN = false>
 LBD T collide_bgk(T* f, const T* acc, const T* prm, T rho0, T* vel, T& ds) {
     T inv_tau = prm[0], rlx_cff1 = T(1.0) - inv_tau, rlx_cff2 = (T(1.0) - T(0.5) * inv_tau);
     T h[10], den;
@@ -175,12 +189,12 @@ LBD T collide_bgk(T* f, const T* acc, const T* prm, T rho0, T* vel, T& ds) {
     forcing<T>(h, acc, den, jx, jy, jz, rlx_cff2, rlx_cff2);
 #pragma unroll
     for (int l = 0; l < Q; ++l) f[l] *= rlx_cff1;
-    project<T, true, DIV>(h, f);
+    project<T, true, DIV, LEAN>(h, f);
     return den;
 }
 
 // forw_euler_TRT, D3Q19.pyx:745-853. prm[0] = 1/tau_even, prm[1] = 1/tau_odd.
-template <class T, bool SH, bool DIV = false>
+template <class T, bool SH, bool DIV = false, bool LEAN = false>
 LBD T collide_trt(T* f, const T* acc, const T* prm, T rho0, T* vel, T& ds) {
     T inv_tau_e = prm[0], inv_tau_o = prm[1];
     T rlx_cff1 = T(1.0) - T(0.5) * inv_tau_o;
@@ -210,12 +224,12 @@ LBD T collide_trt(T* f, const T* acc, const T* prm, T rho0, T* vel, T& ds) {
         f[18 - l] = rlx_cff3 * f[18 - l] - rlx_cff4 * faux;
     }
     f[9] *= (T(1.0) - inv_tau_e);
-    project<T, true, DIV>(h, f);
+    project<T, true, DIV, LEAN>(h, f);
     return den;
 }
 
 // forw_euler_regul, D3Q19.pyx:859-940
-template <class T, bool SH, bool DIV = false>
+template <class T, bool SH, bool DIV = false, bool LEAN = false>
 LBD T collide_reg(T* f, const T* acc, const T* prm, T rho0, T* vel, T& ds) {
     T inv_tau = prm[0], rlx_cff1 = T(1.0) - inv_tau, rlx_cff2 = (T(1.0) - T(0.5) * inv_tau);
     T he[10], h[10];
@@ -236,18 +250,18 @@ LBD T collide_reg(T* f, const T* acc, const T* prm, T rho0, T* vel, T& ds) {
 #pragma unroll
     for (int m = 0; m < 10; ++m) h[m] += inv_tau * he[m];
     forcing<T>(h, acc, den, jx, jy, jz, rlx_cff2, rlx_cff2);
-    project<T, false, DIV>(h, f);
+    project<T, false, DIV, LEAN>(h, f);
     return den;
 }
 
 // DIV: the projection's quotients are corrected (the FP32-shifted variant:
 // its error against FP64 on a 512x128x128 duct drops from 2.4e-5 to 1.2e-6;
 // FP16 storage, whose error is its storage, keeps the plain products)
-template <int RLX, class T, bool SH, bool DIV = false>
+template <int RLX, class T, bool SH, bool DIV = false, bool LEAN = false>
 LBD T collide(T* f, const T* acc, const T* prm, T rho0, T* vel, T& ds) {
-    if constexpr (RLX == BGK) return collide_bgk<T, SH, DIV>(f, acc, prm, rho0, vel, ds);
-    else if constexpr (RLX == TRT) return collide_trt<T, SH, DIV>(f, acc, prm, rho0, vel, ds);
-    else return collide_reg<T, SH, DIV>(f, acc, prm, rho0, vel, ds);
+    if constexpr (RLX == BGK) return collide_bgk<T, SH, DIV, LEAN>(f, acc, prm, rho0, vel, ds);
+    else if constexpr (RLX == TRT) return collide_trt<T, SH, DIV, LEAN>(f, acc, prm, rho0, vel, ds);
+    else return collide_reg<T, SH, DIV, LEAN>(f, acc, prm, rho0, vel, ds);
 }
 
 // ---- Zou-He faces ----------------------------------------------------------
