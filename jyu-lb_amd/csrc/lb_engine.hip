@@ -537,19 +537,120 @@ __global__ void k_sync_in(const uint8_t* hphase, const double* hden, const doubl
     if ((threadIdx.x & 63) == 0 && w) atomicOr(flags, w);
 }
 
-// den/vel of the fluid sites into the staged host fields (the SOLID sites
-// keep the host's values: the reference never writes them)
-__global__ void k_scatter_fluid(const uint32_t* mask, const double* den, const double* vel, double* hden,
-                                double* hvel, Dims d, uint32_t nq) {
+// The same straight from pinned host memory, without staging: per wave one
+// row's 64 sites, whose phase and acceleration are read once, in whole lines
+// (57 GB/s, the copy engine's rate; three loads of stride 24 bytes would read
+// every line three times, as nothing caches host memory). Density and velocity
+// are read where a step needs the host's: of SOLID sites here, of moving
+// sites by k_host_rho. The fluid sites' are overwritten by the call's last
+// step, so they stay on the host: 25 of 57 bytes per cell cross the bus.
+template <class TC>
+__global__ __launch_bounds__(256) void k_host_in(const uint8_t* hphase, const double* hden, const double* hvel,
+                                                 const double* hacc, const uint8_t* phase, double* den, double* vel,
+                                                 TC* acc, Dims d, uint32_t nq, unsigned int* flags) {
+    __shared__ double row[4][192];
+    const uint32_t c = blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    double* const r = row[threadIdx.x >> 6];
+    int i = 0, j = 0, k = d.nz;
+    if (c < nq) decompose(c, d.ny, d.nzp, i, j, k);
+    const bool in = c < nq && k < d.nz;
+    const int n3 = c < nq ? 3 * min(64, d.nz - (k - lane)) : 0;  // doubles of this wave's sites
+    const int64_t o = c < nq ? host_idx(d, i, j, k - lane) : 0;  // its first site
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        if (lane + 64 * a < n3) r[lane + 64 * a] = hacc[3 * o + lane + 64 * a];
+    const bool fluid = in && phase[c] != SOLID;
+    unsigned fl = in && (hphase[o + lane] != SOLID) != fluid ? SYNC_PHASE : 0u;
+    __syncthreads();
+    double v[3] = {0.0, 0.0, 0.0};
+    if (in)
+        for (int a = 0; a < 3; ++a) v[a] = r[3 * lane + a];
+    if (v[0] != 0.0 || v[1] != 0.0 || v[2] != 0.0) fl |= SYNC_ACC;
+    if (c < nq)
+        for (int a = 0; a < 3; ++a) acc[(int64_t)a * nq + c] = (TC)v[a];
+    __syncthreads();
+    const unsigned long long solid = __ballot(in && !fluid);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        if (lane + 64 * a < n3 && (solid >> ((lane + 64 * a) / 3) & 1ull))
+            r[lane + 64 * a] = hvel[3 * o + lane + 64 * a];
+    __syncthreads();
+    if (in && !fluid) {
+        den[c] = hden[o + lane];
+        for (int a = 0; a < 3; ++a) {
+            const double w = r[3 * lane + a];
+            if (w != vel[(int64_t)a * nq + c]) fl |= SYNC_WALLS;
+            vel[(int64_t)a * nq + c] = w;
+        }
+    }
+    const unsigned w = (__ballot((fl & SYNC_PHASE) != 0) ? SYNC_PHASE : 0u) |
+                       (__ballot((fl & SYNC_WALLS) != 0) ? SYNC_WALLS : 0u) |
+                       (__ballot((fl & SYNC_ACC) != 0) ? SYNC_ACC : 0u);
+    if (lane == 0 && w) atomicOr(flags, w);
+}
+// the flags to the host, and cleared for the next call
+__global__ void k_host_flags(unsigned int* flags, unsigned int* host) {
+    *host = *flags;
+    *flags = 0u;
+}
+// densities that Ladd's term reads in the first step
+__global__ void k_host_rho(const uint32_t* cell, uint32_t n, const double* hden, double* den, Dims d) {
+    const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    int i, j, k;
+    decompose(cell[q], d.ny, d.nzp, i, j, k);
+    den[cell[q]] = hden[host_idx(d, i, j, k)];
+}
+// Fluid sites of the outermost layers, whose den/vel the halo pass copies:
+// from the fields into the staged host layout (stage), or from there into the
+// host fields.
+__global__ void k_host_shell(const uint32_t* mask, const double* den, const double* vel, double* sden, double* svel,
+                             double* hden, double* hvel, Dims d, uint32_t nq, bool stage) {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nq || !(mask[c] & M_FLUID)) return;
+    if (c >= nq) return;
     int i, j, k;
     decompose(c, d.ny, d.nzp, i, j, k);
+    if (i > 0 && i < d.nx - 1 && j > 0 && j < d.ny - 1 && k > 0 && k < d.nz - 1) return;
+    if (!(mask[c] & M_FLUID)) return;
     const int64_t o = host_idx(d, i, j, k);
-    hden[o] = den[c];
-    hvel[3 * o] = vel[c];
-    hvel[3 * o + 1] = vel[nq + c];
-    hvel[3 * o + 2] = vel[2 * (int64_t)nq + c];
+    if (stage) {
+        sden[o] = den[c];
+        for (int a = 0; a < 3; ++a) svel[3 * o + a] = vel[(int64_t)a * nq + c];
+    } else {
+        hden[o] = sden[o];
+        for (int a = 0; a < 3; ++a) hvel[3 * o + a] = svel[3 * o + a];
+    }
+}
+
+// den/vel of the fluid sites into the staged host fields, or into the host
+// fields themselves where those are pinned (the SOLID sites keep the host's
+// values: the reference never writes them)
+// Per wave one row's 64 sites; the velocities go through LDS, so that each
+// store of the wave covers one run of memory (into host memory 54 GB/s;
+// three stores of stride 24 bytes 46).
+__global__ __launch_bounds__(256) void k_scatter_fluid(const uint32_t* mask, const double* den, const double* vel,
+                                                       double* hden, double* hvel, Dims d, uint32_t nq) {
+    __shared__ double row[4][192];
+    const uint32_t c = blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    double* const r = row[threadIdx.x >> 6];
+    const bool fluid = c < nq && (mask[c] & M_FLUID) != 0;
+    int64_t o = 0;  // of the wave's first site
+    if (c < nq) {
+        int i, j, k;
+        decompose(c, d.ny, d.nzp, i, j, k);
+        o = host_idx(d, i, j, k - lane);
+    }
+    if (fluid) {
+        hden[o + lane] = den[c];
+        for (int a = 0; a < 3; ++a) r[3 * lane + a] = vel[(int64_t)a * nq + c];
+    }
+    const unsigned long long live = __ballot(fluid);
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        if (live >> ((lane + 64 * a) / 3) & 1ull) hvel[3 * o + lane + 64 * a] = r[lane + 64 * a];
 }
 
 // _enforce_den_vel_per_sym_bc (isothermal.pyx:582-686) on the staged host
@@ -710,6 +811,9 @@ struct lb_solver {
     uint8_t* st_phase = nullptr;
     double *st_den = nullptr, *st_vel = nullptr, *st_acc = nullptr;
     int64_t ncnt = 0;
+    bool h_pinned = false;             // kernels read and write the host fields themselves (k_host_in)
+    unsigned int* in_flags = nullptr;  // SYNC_* of k_host_in, zero between calls, and their place on the host
+    unsigned int* h_flags = nullptr;
     // FP16 storage guard: steps between checks of the stored magnitudes, steps
     // since the last check, and whether the scale was chosen automatically
     uint32_t f16_check = 64, f16_since = 0;
@@ -1657,6 +1761,8 @@ int lb_destroy(lb_solver* s) {
                     s->mov_cell, s->mov_word, s->den2, s->tabc, s->tabw, s->f2, s->prev, s->dseed, s->st_phase, s->st_den, s->st_vel, s->st_acc};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    (void)hipFree(s->in_flags);
+    (void)hipHostFree(s->h_flags);
     for (int f = 0; f < 6; ++f) {
         if (s->fden[f]) (void)hipFree(s->fden[f]);
         if (s->fvel[f]) (void)hipFree(s->fvel[f]);
@@ -2344,6 +2450,20 @@ int lb_host_free(void* ptr) {
     return LB_OK;
 }
 
+// Whether the device reaches host memory [p, p + n) at its host address
+// (lb_host_alloc's does; a caller may bind any memory).
+static bool pinned(const void* p, size_t n) {
+    for (const char* q : {(const char*)p, (const char*)p + n - 1}) {
+        void* dev = nullptr;
+        if (hipHostGetDevicePointer(&dev, const_cast<char*>(q), 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (dev != q) return false;
+    }
+    return true;
+}
+
 int lb_bind_host_fields(lb_solver* s, uint8_t* phase, double* den, double* vel, double* acc) {
     if (!s) return fail(LB_EINVAL, "null handle");
     if (s->stream) HIPCHK(hipStreamSynchronize(s->stream));
@@ -2363,6 +2483,13 @@ int lb_bind_host_fields(lb_solver* s, uint8_t* phase, double* den, double* vel, 
             return rc;
     }
     if (!s->acc && (rc = dalloc(s, &s->acc, (size_t)3 * s->nq * tc_size(s->prec)))) return rc;
+    if (!s->in_flags) {
+        if ((rc = dalloc(s, (void**)&s->in_flags, 4))) return rc;
+        HIPCHK(hipMemset(s->in_flags, 0, 4));
+    }
+    if (!s->h_flags && (rc = lb_host_alloc(4, (void**)&s->h_flags))) return rc;
+    s->h_pinned = pinned(phase, (size_t)ncnt) && pinned(den, (size_t)ncnt * 8) && pinned(vel, (size_t)ncnt * 24) &&
+                  pinned(acc, (size_t)ncnt * 24);
     s->ncnt = ncnt;
     s->h_phase = phase;
     s->h_den = den;
@@ -2377,30 +2504,42 @@ static bool has_halo_faces(const lb_solver* s) {
     return false;
 }
 
+// The den/vel halo pass on the fields hden and hvel, in the host layout
+static int halo_faces(lb_solver* s, double* hden, double* hvel) {
+    const int64_t n[3] = {(int64_t)s->d.ny * s->d.nz, (int64_t)s->NI * s->d.nz, (int64_t)s->NI * s->NJ};
+    for (int a = 0; a < 3; ++a) {
+        if (s->cfg.bc[2 * a] != PERIODIC && s->cfg.bc[2 * a] != SYMMETRIC && s->cfg.bc[2 * a + 1] != PERIODIC &&
+            s->cfg.bc[2 * a + 1] != SYMMETRIC)
+            continue;
+        k_halo_dv<<<(unsigned)((n[a] + 255) / 256), 256, 0, s->stream>>>(hden, hvel, s->d, a);
+    }
+    HIPCHK(hipGetLastError());
+    return LB_OK;
+}
+
 // den/vel of the fluid sites into the staged host fields, optionally the
 // den/vel halo pass there
 static int scatter_staged(lb_solver* s, bool halo) {
     k_scatter_fluid<<<blocks_for(s->nq, 256), 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->st_den, s->st_vel,
                                                                    s->d, s->nq);
     HIPCHK(hipGetLastError());
-    if (halo) {
-        const int64_t n[3] = {(int64_t)s->d.ny * s->d.nz, (int64_t)s->NI * s->d.nz, (int64_t)s->NI * s->NJ};
-        for (int a = 0; a < 3; ++a) {
-            if (s->cfg.bc[2 * a] != PERIODIC && s->cfg.bc[2 * a] != SYMMETRIC && s->cfg.bc[2 * a + 1] != PERIODIC &&
-                s->cfg.bc[2 * a + 1] != SYMMETRIC)
-                continue;
-            k_halo_dv<<<(unsigned)((n[a] + 255) / 256), 256, 0, s->stream>>>(s->st_den, s->st_vel, s->d, a);
-        }
-        HIPCHK(hipGetLastError());
-    }
+    if (halo) return halo_faces(s, s->st_den, s->st_vel);
     return LB_OK;
 }
 
-static int halo_only(lb_solver* s) {
-    const int64_t n[3] = {(int64_t)s->d.ny * s->d.nz, (int64_t)s->NI * s->d.nz, (int64_t)s->NI * s->NJ};
-    for (int a = 0; a < 3; ++a)
-        k_halo_dv<<<(unsigned)((n[a] + 255) / 256), 256, 0, s->stream>>>(s->st_den, s->st_vel, s->d, a);
-    HIPCHK(hipGetLastError());
+// What a call's host fields said (SYNC_* flags): refused, or taken.
+static int host_inputs(lb_solver* s, unsigned int hf) {
+    if (hf & SYNC_PHASE)
+        return fail(LB_ESTATE, "the phase field was changed after finalize_init; the engine builds its links "
+                    "from the phase at finalize_init, so phase edits after it are not supported");
+    if (hf & SYNC_WALLS) {  // wall velocities changed: moving-wall flags and Ladd table
+        int rc = build_mask(s, true);
+        if (rc) return rc;
+        int64_t nf, nm;
+        if ((rc = count_mask(s, &nf, &nm))) return rc;
+        s->moving = nm > 0;
+    }
+    s->acc_on = (hf & SYNC_ACC) != 0;
     return LB_OK;
 }
 
@@ -2427,18 +2566,7 @@ static int load_host_fields(lb_solver* s) {
     unsigned int hf = 0;
     HIPCHK(hipMemcpyAsync(&hf, flags, 4, hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
-    if (hf & SYNC_PHASE)
-        return fail(LB_ESTATE, "the phase field was changed after finalize_init; the engine builds its links "
-                    "from the phase at finalize_init, so phase edits after it are not supported");
-    if (hf & SYNC_WALLS) {  // wall velocities changed: moving-wall flags and Ladd table
-        int rc = build_mask(s, true);
-        if (rc) return rc;
-        int64_t nf, nm;
-        if ((rc = count_mask(s, &nf, &nm))) return rc;
-        s->moving = nm > 0;
-    }
-    s->acc_on = (hf & SYNC_ACC) != 0;
-    return LB_OK;
+    return host_inputs(s, hf);
 }
 
 int lb_load_host_fields(lb_solver* s) {
@@ -2449,12 +2577,61 @@ int lb_load_host_fields(lb_solver* s) {
     return load_host_fields(s);
 }
 
+// load_host_fields from pinned host fields (k_host_in).
+static int load_pinned(lb_solver* s) {
+    if (tc_size(s->prec) == 8)
+        k_host_in<double><<<blocks_for(s->nq, 256), 256, 0, s->stream>>>(s->h_phase, s->h_den, s->h_vel, s->h_acc, s->phase,
+                                                                       s->den, s->vel, (double*)s->acc, s->d, s->nq,
+                                                                       s->in_flags);
+    else
+        k_host_in<float><<<blocks_for(s->nq, 256), 256, 0, s->stream>>>(s->h_phase, s->h_den, s->h_vel, s->h_acc, s->phase,
+                                                                      s->den, s->vel, (float*)s->acc, s->d, s->nq,
+                                                                      s->in_flags);
+    k_host_flags<<<1, 1, 0, s->stream>>>(s->in_flags, s->h_flags);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s->stream));
+    const int rc = host_inputs(s, *(volatile unsigned int*)s->h_flags);
+    if (rc) return rc;
+    if (s->moving) {
+        k_host_rho<<<blocks_for(s->nmov, 256), 256, 0, s->stream>>>(s->mov_cell, s->nmov, s->h_den, s->den, s->d);
+        HIPCHK(hipGetLastError());
+    }
+    return LB_OK;
+}
+
+// lb_evolve_host on pinned host fields: read by k_host_in and written, with
+// the halo pass, by the kernels themselves. Nothing is written to them before
+// the last step has run and the FP16 guard has passed, so the layers of step
+// T-1 that the halo pass copies wait in the staged fields.
+static int evolve_pinned(lb_solver* s, uint32_t steps) {
+    int rc = load_pinned(s);
+    if (rc) return rc;
+    const bool halo = has_halo_faces(s), shell = halo && steps >= 2;
+    const unsigned nb = blocks_for(s->nq, 256);
+    if (shell) {
+        if ((rc = evolve_steps(s, steps - 1))) return rc;
+        k_host_shell<<<nb, 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->st_den, s->st_vel, s->h_den, s->h_vel, s->d,
+                                                s->nq, true);
+    }
+    if ((rc = evolve_steps(s, halo ? 1 : steps))) return rc;
+    if (s->prec == LB_FP16_STORAGE && (rc = fp16_guard(s))) return rc;  // no silent inf in the fields
+    if (shell)
+        k_host_shell<<<nb, 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->st_den, s->st_vel, s->h_den, s->h_vel, s->d,
+                                                s->nq, false);
+    if (halo && (rc = halo_faces(s, s->h_den, s->h_vel))) return rc;
+    k_scatter_fluid<<<nb, 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->h_den, s->h_vel, s->d, s->nq);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s->stream));
+    return LB_OK;
+}
+
 int lb_evolve_host(lb_solver* s, uint32_t steps) {
     if (!s) return fail(LB_EINVAL, "null handle");
     if (!s->finalized) return fail(LB_ESTATE, "Finalize solver initialization before calling evolve");
     if (!s->h_phase) return fail(LB_ESTATE, "no host fields bound (lb_bind_host_fields)");
     inputs_changed(s);
     if (s->nfluid < 1 || steps == 0) return LB_OK;
+    if (s->h_pinned) return evolve_pinned(s, steps);
     int rc = load_host_fields(s);
     if (rc) return rc;
     // Isothermal.evolve: the halo den/vel pass precedes every step, so after
@@ -2463,7 +2640,7 @@ int lb_evolve_host(lb_solver* s, uint32_t steps) {
     if (halo && steps >= 2) {
         if ((rc = evolve_steps(s, steps - 1))) return rc;
         if ((rc = scatter_staged(s, true))) return rc;
-    } else if (halo && (rc = halo_only(s))) {
+    } else if (halo && (rc = halo_faces(s, s->st_den, s->st_vel))) {
         return rc;
     }
     if ((rc = evolve_steps(s, halo ? 1 : steps))) return rc;
@@ -2480,6 +2657,15 @@ int lb_store_host_fields(lb_solver* s, int halo_pass) {
     if (!s) return fail(LB_EINVAL, "null handle");
     if (!s->h_phase) return fail(LB_ESTATE, "no host fields bound (lb_bind_host_fields)");
     const int64_t n = s->ncnt;
+    if (s->h_pinned) {
+        k_scatter_fluid<<<blocks_for(s->nq, 256), 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->h_den, s->h_vel, s->d,
+                                                                       s->nq);
+        HIPCHK(hipGetLastError());
+        const int rc = halo_pass != 0 && has_halo_faces(s) ? halo_faces(s, s->h_den, s->h_vel) : LB_OK;
+        if (rc) return rc;
+        HIPCHK(hipStreamSynchronize(s->stream));
+        return LB_OK;
+    }
     // the SOLID sites and halos keep the host's values
     HIPCHK(hipMemcpyAsync(s->st_den, s->h_den, (size_t)n * 8, hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(s->st_vel, s->h_vel, (size_t)n * 24, hipMemcpyHostToDevice, s->stream));
