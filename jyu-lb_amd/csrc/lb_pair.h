@@ -16,10 +16,10 @@
 // Only the first step of the rim is computed twice (by this tile and by its
 // neighbour), so two steps move little more than one step's bytes. Results
 // are bit-identical to single steps. Measured (ms per step, single / paired):
-// 256^3 FP64 0.894 / 0.593 (a pair moves 6.6 GB past L2, 5.5 TB/s: the rims'
+// 256^3 FP64 0.894 / 0.570 (a pair moves 6.6 GB past L2, 5.8 TB/s: the rims'
 // lines, of which L2 catches about half, are what is left), FP32 0.451 /
-// 0.323 and FP16 0.274 / 0.277 (bound by the collisions' instructions);
-// 512x128x128 duct FP64 0.433 / 0.323; 32x34x8 channel 0.0185 / 0.0045.
+// 0.315 and FP16 0.274 / 0.277 (bound by the collisions' instructions);
+// 512x128x128 duct FP64 0.433 / 0.299; 32x34x8 channel 0.0185 / 0.0042.
 //
 // LDS. A population with c_i = -1 is needed in the iteration it is made in,
 // one with c_i = 0 in the next, one with c_i = +1 in the one after, so the
@@ -356,9 +356,12 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
             uint64_t step = (uint64_t)psb;
             uint32_t o = own;
             asm volatile("" : "+s"(step), "+v"(o));  // not multiplied out, nor widened, ahead of the loop
+            // Plain stores: L2 joins the lines that two tiles share. With
+            // non-temporal ones 256^3 FP64 ran 0.615 ms per step (plain
+            // 0.572) and tiles that split lines 0.968 (33x12x32; 0.751).
 #pragma unroll
             for (int sl = 0; sl < Q; ++sl) {
-                st_stream<(LB_NT_MASK & 2) != 0>((TS*)(uniform_ptr(G) + o), to_ts<P>(h[opp(sl)], p.scale));
+                *(TS*)(uniform_ptr(G) + o) = to_ts<P>(h[opp(sl)], p.scale);
                 G += step;
             }
         }
