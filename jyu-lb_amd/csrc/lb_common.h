@@ -335,11 +335,14 @@ struct PairParams {
     double* rho_out;
 };
 constexpr int PAIR_WALLS = 4;
-constexpr int PAIR_MOVING = 1, PAIR_FULL = 2;
+constexpr int PAIR_MOVING = 1, PAIR_FULL = 2, PAIR_SPARSE = 4;
 // Columns of a tile, rim included, one per thread. FP64 arithmetic holds the
 // next plane's populations and a collision in 256 VGPRs (2 waves per SIMD);
 // FP32 arithmetic in 168 (3 waves per SIMD).
 constexpr int pair_threads(int prec) { return prec == LB_FP64 || prec == LB_FP32_STORAGE ? 512 : 768; }
+// Sparse layout: cells of a tile with its rim and one more column around it,
+// whose compact indices the first step's gather looks up; two per thread.
+constexpr int pair_cells(int prec) { return 2 * pair_threads(prec); }
 
 // Launchers of the per-precision kernels, defined in lb_kernels.h and
 // instantiated once per precision P in its own translation unit (lb_inst.hip,

@@ -1529,13 +1529,24 @@ static void layout_defaults(lb_solver* s, int layout) {
     }
 }
 
-// Whether a dense layout steps in pairs (k_pair) where a call has two steps
-// left: not with a symmetric x face (the sweep along i does not mirror), nor
+// Whether steps are paired (k_pair) where a call has two of them left: not with a symmetric x face (the sweep along i does not mirror), nor
 // where three planes of populations exceed the kernel's 32-bit offsets, nor
 // where LB_SP_PULL asks for single steps of one kind. rs and ps are set.
+//
+// In the sparse layout (nfluid is set) pairs are a candidate, which tune_pair
+// times: solid cells are columns that idle, every first step looks its
+// upstream sites up, and small lattices wait for that chain. Measured (ms per
+// step, single / paired): random spheres of 20% solid FP64 384x192x192 0.643 /
+// 0.492, 192^3 0.320 / 0.256, 128^3 0.0848 / 0.0803, 64^3 0.0149 / 0.0150;
+// FP32 256x128x128 0.0898 / 0.0896, 64^3 0.0085 / 0.0123; 40% solid FP64
+// 256^3 0.578 / 0.641. FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 /
+// 0.561) stay single.
 static bool pair_wanted(const lb_solver* s) {
-    if (s->sparse || s->sp_pull >= 0 || s->pair == 0) return false;
+    if (s->sp_pull >= 0 || s->pair == 0) return false;
     if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
+    if (s->sparse)
+        return s->pair > 0 || (s->autotune && (s->prec == LB_FP64 || s->prec == LB_FP32_SHIFTED) &&
+                               s->nfluid >= (1 << 19) && s->nfluid * 10 >= s->ncell * 7);
     const uint64_t ts = ts_size(s->prec);
     return 3 * (uint64_t)s->d.ny * (uint64_t)s->rs * ts + Q * (uint64_t)s->ps * ts < (1ull << 32);
 }
@@ -1572,7 +1583,7 @@ static void pair_tiling(lb_solver* s) {
         q.hj = q.ntj > 1 || perj;
         q.chunk = chunk;
         const int EK = TK + 2 * q.hk, cols = EK * (TJ + 2 * q.hj);
-        if (cols > NT) return;
+        if (cols > NT || (s->sparse && (EK + 2) * (TJ + 2 * q.hj + 2) > pair_cells(s->prec))) return;
         const uint64_t total = (uint64_t)q.ntk * q.ntj * (uint64_t)((d.nx + chunk - 1) / chunk);
         if (total > (1u << 30)) return;
         q.total = (uint32_t)total;
@@ -1605,7 +1616,7 @@ static void pair_tiling(lb_solver* s) {
             const int TK = (d.nz + ntk - 1) / ntk, TK8 = (TK + 7) / 8 * 8;
             if (TK > NT / 3) continue;
             if (ntk > 1 && TK < 20) break;
-            all_of(ntk > 1 ? TK8 : TK);  // tiles start on half a line at least: unaligned ones (37x11x86) ran 256^3 FP64 at 0.886
+            all_of(ntk > 1 && !s->sparse ? TK8 : TK);  // tiles start on half a line at least: unaligned ones (37x11x86) ran 256^3 FP64 at 0.886
         }
     }
     memcpy(best.wall, s->pq.wall, sizeof(best.wall));
@@ -1959,6 +1970,7 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
         if ((rc = layout_arrays(s, layout))) return rc;
     }
     if (s->sparse && (rc = build_sparse(s))) return rc;
+    if (s->sparse) s->pair_on = pair_wanted(s);
     if (s->pair_tune) s->pair_on = true;  // finalized again
     if (s->pair_on) pair_tiling(s);
     if (s->pair_on && s->moving && (rc = pair_walls(s))) return rc;
@@ -1970,7 +1982,8 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
         // collisions bind, it depends: cavities 256^3 FP64 0.928 / 0.648, FP16
         // 0.284 / 0.389, 160^3 FP32 0.118 / 0.132, 64^3 FP64 0.0164 / 0.0171,
         // 48^3 FP64 0.0128 / 0.0102; 64^3 channel FP16 0.0184 / 0.0112.
-        s->pair_tune = s->pair < 0 && s->autotune && (s->moving || s->prec == LB_FP16_STORAGE);
+        // In the sparse layout it depends on the solid too, whose columns idle.
+        s->pair_tune = s->pair < 0 && s->autotune && (s->moving || s->sparse || s->prec == LB_FP16_STORAGE);
         if (s->pair_tune) s->pair_on = false;
         else s->tune = false;  // few single steps are left to tune
     }

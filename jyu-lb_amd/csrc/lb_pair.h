@@ -1,4 +1,4 @@
-// Two fused steps in one pass over the dense population array (k_pair), from
+// Two fused steps in one pass over the population array (k_pair), from
 // the state an even AA step leaves (site y's post-collision population l in
 // its own slot opp(l)) in p.f to the same form in p.f2. Included by
 // lb_kernels.h.
@@ -29,6 +29,14 @@
 // registers. That is 36 values per column: with 512 columns of 8 bytes
 // 144 KiB, one workgroup per CU. The loads of the next plane are issued
 // before the second step computes, so memory works during both collisions.
+//
+// Sparse layout (PAIR_SPARSE). The same sweep over the cells of a tile; only
+// fluid sites load and store. The compact indices around come from LDS too
+// (18 of them per site; the single step reads 9 bytes of codes), a ring of
+// four planes, each loaded an iteration ahead. Tiles' rows start and end
+// anywhere in a line: L2 joins the stores (1.80 GB written for 1.72 GB of
+// populations on 384x192x192 cells of 20% solid). ms per step there, single /
+// paired: FP64 0.643 / 0.492; 256x128x128 0.179 / 0.154.
 #pragma once
 #include <type_traits>
 
@@ -82,8 +90,17 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
     using TS = typename Var<P>::TS;
     using TC = typename Var<P>::TC;
     constexpr bool SH = Var<P>::SH, FULL = (FEAT & PAIR_FULL) != 0, MOV = (FEAT & PAIR_MOVING) != 0;
-    constexpr int NT = pair_threads(P);
+    constexpr bool SP = (FEAT & PAIR_SPARSE) != 0;
+    constexpr int NT = pair_threads(P), NC = pair_cells(P);
+    // The gather's loads that are issued before the first step; the others
+    // follow it, and have the second step's time to arrive. Measured (ms per
+    // step, all 19 first / 14): FP32 256^3 0.322 / 0.300, sparse 256x128x128
+    // 0.103 / 0.090; sparse FP64 384x192x192 0.501 / 0.492; but dense FP64
+    // 256^3, which waits for memory as it is, 0.566 / 0.595.
+    constexpr int FIRST = (P == LB_FP64 && !SP) || (MOV && FULL) ? Q : 14;
+    auto in_part = [](int part, int l) constexpr { return part < 0 || (l < FIRST) == (part == 0); };
     __shared__ TS ring[RING_SLOTS * NT];
+    __shared__ uint32_t idx[SP ? 4 * NC : 1];
 
     // tile and chunk of this workgroup: each XCD takes a contiguous range, so
     // that neighbouring tiles, which read each other's rims, share its L2
@@ -156,7 +173,8 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
     // that counts the stores.) The asm keeps the strides from being
     // multiplied out ahead of the loop, into registers it does not have.
     TS g[Q] = {};
-    auto gather = [&](const char* Fl, const char* F, const char* Fh, int ip, uint32_t m) {
+    auto gather = [&](auto part, const char* Fl, const char* F, const char* Fh, int ip, uint32_t m) {
+        constexpr int PT = decltype(part)::value;
         const bool follow = !perx || (ip > 0 && ip < nx - 1);
         if (!(m & M_FLUID)) return;
         uint32_t sb = (uint32_t)psb, pb = (uint32_t)plane;
@@ -173,7 +191,7 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         if (some) {
 #pragma unroll
             for (int l = 0; l < Q; ++l) {
-                if (l == REST) continue;
+                if (l == REST || !in_part(PT, l)) continue;
                 if (FULL && (CJ[l] || CK[l])) {  // the mirrored population's slot
                     const bool y = CJ[l] && sy[CJ[l] + 1], z = CK[l] && sz[CK[l] + 1];
                     uint32_t d = 0;
@@ -188,12 +206,70 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         }
 #pragma unroll
         for (int l = 0; l < Q; ++l)
-            g[l] = *(const TS*)((CI[l] > 0 ? bl : CI[l] < 0 ? bh : b0) + off[l]);
+            if (in_part(PT, l)) g[l] = *(const TS*)((CI[l] > 0 ? bl : CI[l] < 0 ? bh : b0) + off[l]);
         if (some && !follow) {
 #pragma unroll
             for (int l = 0; l < Q; ++l)
-                if (CI[l] != 0 && (m & (1u << l))) g[l] = *(const TS*)(b0 + (own + (uint32_t)l * sb));
+                if (CI[l] != 0 && in_part(PT, l) && (m & (1u << l))) g[l] = *(const TS*)(b0 + (own + (uint32_t)l * sb));
         }
+    };
+    // The same in the sparse layout: the compact indices of the planes around
+    // are in LDS (a ring of four planes, I0 the plane before). 32-bit element
+    // offsets reach the whole array (19 * ps < 2^32).
+    const int EX = EK + 2, xc = (jj + 1) * EX + kk + 1;
+    uint32_t nN = 0, nA = 0, nB = 0;  // own compact index in planes i + 1, i, i - 1
+    auto gather_sp = [&](auto part, const uint32_t* I0, const uint32_t* I1, const uint32_t* I2, uint32_t m) {
+        constexpr int PT = decltype(part)::value;
+        if (!(m & M_FLUID)) return;
+        uint32_t np = (uint32_t)p.ps;
+        asm volatile("" : "+s"(np));
+        const TS* const b = uniform_ptr((const TS*)p.f);
+        nN = I1[xc];
+#pragma unroll
+        for (int l = 0; l < Q; ++l) {
+            if (!in_part(PT, l)) continue;
+            uint32_t e = (uint32_t)opp(l) * np;
+            if (l == REST) {
+                e += nN;
+            } else {
+                e += (CI[l] > 0 ? I0 : CI[l] < 0 ? I2 : I1)[xc - CJ[l] * EX - CK[l]];
+                if (FULL && (CJ[l] || CK[l])) {
+                    const bool y = CJ[l] && sy[CJ[l] + 1], z = CK[l] && sz[CK[l] + 1];
+                    uint32_t d = 0;
+                    if (y) d = (uint32_t)(l - mirror(l, 1)) * np;
+                    if (z) d = (uint32_t)(l - mirror(l, 2)) * np;
+                    if (y && z) d = (uint32_t)(l - mirror(mirror(l, 2), 1)) * np;
+                    e += d;
+                }
+                const uint32_t mine = (uint32_t)l * np + nN;
+                e = m & (1u << l) ? mine : e;
+            }
+            g[l] = b[e];
+        }
+    };
+    // Cells of those planes that this thread keeps: clamped to the lattice
+    // beyond a wall or a symmetric face, where the mirrored populations are.
+    uint32_t cell[2] = {0, 0}, cv[2] = {0, 0};
+    if (SP) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int y = (t + e * NT) / EX, z = (t + e * NT) - y * EX;
+            int cj = j0 - q.hj - 1 + y, ck = k0 - q.hk - 1 + z;
+            if (pery) cj = cj < 0 ? cj + ny : cj >= ny ? cj - ny : cj;
+            if (perz) ck = ck < 0 ? ck + nz : ck >= nz ? ck - nz : ck;
+            cj = min(max(cj, 0), ny - 1);
+            ck = min(max(ck, 0), nz - 1);
+            cell[e] = (uint32_t)cj * (uint32_t)p.d.nzp + (uint32_t)ck;
+        }
+    }
+    auto load_idx = [&](int i) {
+        const uint32_t* const b = uniform_ptr(p.cidx + (uint32_t)max(wrapx(i), 0) * cplane);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) cv[e] = b[cell[e]];
+    };
+    auto keep_idx = [&](int slot) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) idx[slot * NC + e * NT + t] = cv[e];
     };
     // One collision, on the streamed populations f of the site (ip, jw, kw).
     // What is loaded in a branch is waited for there: a wait behind it would
@@ -241,6 +317,7 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
 #pragma unroll
         for (int l = 0; l < Q; ++l) asm volatile("" : "+v"(g[l]));
         if (MOV) asm volatile("" : "+v"(wN), "+v"(rhoN));
+        if (SP) asm volatile("" : "+v"(cv[0]), "+v"(cv[1]));
     };
 
     // lattice planes of i - 1, i, i + 1, their places in p.f and their masks
@@ -251,7 +328,26 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
     double dB = 0.0, dA = 0.0;                             // density of planes i - 1, i
     TS r0 = TS(0), m1 = TS(0), p1 = TS(0), p2 = TS(0);  // plane i - 1: rest, l = 2, l = 16; plane i - 2: l = 16
     if (MOV) load_ladd(ip, mA);
-    gather(place(wrapx(i0 - 2)), FA, FN, ip, mA);
+    const std::integral_constant<int, -1> all;
+    const std::integral_constant<int, 0> part0;
+    const std::integral_constant<int, 1> part1;
+    if constexpr (SP) {
+        load_idx(i0 - 2);
+        keep_idx(3);
+        load_idx(i0 - 1);
+        keep_idx(0);
+        load_idx(i0);
+        keep_idx(1);
+        load_idx(i0 + 1);
+        keep_idx(2);
+        lds_barrier();
+        gather_sp(all, idx + 3 * NC, idx, idx + NC, mA);
+        nA = nN;
+        load_idx(i0 + 2);
+        lds_barrier();
+    } else {
+        gather(all, place(wrapx(i0 - 2)), FA, FN, ip, mA);
+    }
     arrive();
     wA = wN;
     rho = rhoN;
@@ -265,7 +361,16 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         const char* const FNN = place(ipNN);
         uint32_t mNN = mask_of(ipNN);
         if (MOV) load_ladd(ipN, mN);
-        if (i < i1) gather(FA, FN, FNN, ipN, mN);
+        // the gather of plane i + 1, one part at a time
+        const int s0 = i - i0 + 1;  // ring plane of i in idx
+        auto load_next = [&](auto part) {
+            if (i >= i1) return;
+            if constexpr (SP)
+                gather_sp(part, idx + (s0 & 3) * NC, idx + (s0 + 1 & 3) * NC, idx + (s0 + 2 & 3) * NC, mN);
+            else
+                gather(part, FA, FN, FNN, ipN, mN);
+        };
+        load_next(part0);
         __builtin_amdgcn_sched_barrier(0);
 
         // ---- first step, plane i ----
@@ -290,7 +395,11 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
                 d[ring_slot(l) * NT] = to_ts<P>(f[l], p.scale);
             }
         }
+        if (SP) keep_idx(s0 + 3 & 3);
         lds_barrier();
+        if (SP) load_idx(i + 4);
+        load_next(part1);
+        __builtin_amdgcn_sched_barrier(0);
         // ---- second step, plane i - 1 ----
         const bool second = i > i0 && inner && (mB & M_FLUID);
         TC h[Q];
@@ -352,9 +461,9 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         arrive();
         asm volatile("" : "+v"(mNN));
         if (second) {
-            char* G = (char*)p.f2 + (int64_t)ipB * plane;
+            char* G = (char*)p.f2 + (SP ? 0 : (int64_t)ipB * plane);
             uint64_t step = (uint64_t)psb;
-            uint32_t o = own;
+            uint32_t o = SP ? nB * (uint32_t)sizeof(TS) : own;
             asm volatile("" : "+s"(step), "+v"(o));  // not multiplied out, nor widened, ahead of the loop
             // Plain stores: L2 joins the lines that two tiles share. With
             // non-temporal ones 256^3 FP64 ran 0.615 ms per step (plain
@@ -375,6 +484,8 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         ipN = ipNN;
         FA = FN;
         FN = FNN;
+        nB = nA;
+        nA = nN;
         wB = wA;
         wA = wN;
         rho = rhoN;
@@ -386,20 +497,27 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
     }
 }
 
-template <int P, int RLX>
+template <int P, int RLX, int LAYOUT>
 static void launch_pair_feat(const StepParams& p, const PairParams& q, int feat, hipStream_t st) {
     const unsigned grid = (q.total + 7) / 8 * 8;
-    if (feat == 0) k_pair<P, RLX, 0><<<grid, pair_threads(P), 0, st>>>(p, q);
-    else if (feat == PAIR_MOVING) k_pair<P, RLX, PAIR_MOVING><<<grid, pair_threads(P), 0, st>>>(p, q);
-    else if (feat == PAIR_FULL) k_pair<P, RLX, PAIR_FULL><<<grid, pair_threads(P), 0, st>>>(p, q);
-    else k_pair<P, RLX, PAIR_MOVING | PAIR_FULL><<<grid, pair_threads(P), 0, st>>>(p, q);
+    constexpr int NT = pair_threads(P);
+    if (feat == 0) k_pair<P, RLX, LAYOUT><<<grid, NT, 0, st>>>(p, q);
+    else if (feat == PAIR_MOVING) k_pair<P, RLX, LAYOUT | PAIR_MOVING><<<grid, NT, 0, st>>>(p, q);
+    else if (feat == PAIR_FULL) k_pair<P, RLX, LAYOUT | PAIR_FULL><<<grid, NT, 0, st>>>(p, q);
+    else k_pair<P, RLX, LAYOUT | PAIR_MOVING | PAIR_FULL><<<grid, NT, 0, st>>>(p, q);
+}
+
+template <int P, int RLX>
+static void launch_pair_layout(const StepParams& p, const PairParams& q, int feat, hipStream_t st) {
+    if (p.cidx) launch_pair_feat<P, RLX, PAIR_SPARSE>(p, q, feat, st);
+    else launch_pair_feat<P, RLX, 0>(p, q, feat, st);
 }
 
 template <int P>
 void launch_pair_rlx(const StepParams& p, const PairParams& q, int rlx, int feat, hipStream_t st) {
-    if (rlx == BGK) launch_pair_feat<P, BGK>(p, q, feat, st);
-    else if (rlx == TRT) launch_pair_feat<P, TRT>(p, q, feat, st);
-    else launch_pair_feat<P, REGUL>(p, q, feat, st);
+    if (rlx == BGK) launch_pair_layout<P, BGK>(p, q, feat, st);
+    else if (rlx == TRT) launch_pair_layout<P, TRT>(p, q, feat, st);
+    else launch_pair_layout<P, REGUL>(p, q, feat, st);
 }
 
 }  // namespace lb

@@ -1,4 +1,4 @@
-"""Paired steps (two fused steps per pass over the dense array, k_pair) against
+"""Paired steps (two fused steps per pass over the population array, k_pair) against
 the reference's fixtures and against single steps: every boundary kind, tiles
 whose edges fall anywhere, and every count of steps."""
 import glob
@@ -19,7 +19,7 @@ def _solver_cls():
     return Solver
 
 
-@pytest.mark.parametrize("layout", ["rows", "soa"])
+@pytest.mark.parametrize("layout", ["rows", "soa", "sparse"])
 @pytest.mark.parametrize("tile", ["", "5,3,2", "3,4,1"], ids=["auto", "5x3x2", "3x4x1"])
 @pytest.mark.parametrize("path", GOLD, ids=[os.path.basename(p)[:-4] for p in GOLD])
 def test_pairs_bit_exact(path, tile, layout, monkeypatch):
@@ -43,11 +43,11 @@ def test_pairs_bit_exact(path, tile, layout, monkeypatch):
         np.testing.assert_array_equal(b, a, err_msg=f"{sc['name']} {k} tile {tile}")
 
 
-def _run(lat, bc, precision, rlx, steps, walls, seed):
+def _run(lat, bc, precision, rlx, steps, walls, seed, layout="rows", solid=0.04):
     rng = np.random.default_rng(seed)
     s = _solver_cls()(np.array(lat, dtype=np.int32), rlx, 0.05, np.array([1e-5, 2e-5, -1e-5]),
-                      np.array(bc, dtype=np.int32), precision=precision, layout="rows")
-    phase = (rng.random(lat) > 0.04).astype(np.uint8)
+                      np.array(bc, dtype=np.int32), precision=precision, layout=layout)
+    phase = (rng.random(lat) > solid).astype(np.uint8)
     s.get_phase()[...] = phase
     s.get_den()[...] = 1.0 + 0.01 * rng.standard_normal(lat)
     s.get_vel()[...] = 0.01 * rng.standard_normal(lat + (3,))
@@ -86,5 +86,28 @@ def test_pairs_equal_single_steps(lat, bc, tile, walls, precision, monkeypatch):
             monkeypatch.setenv("LB_PAIR_TILE", tile)
         print(f"pairs {pair}: {lat} {bc} tile {tile or 'auto'} walls {walls} {precision}", flush=True)
         out.append(_run(lat, bc, precision, 1, (2, 7, 1, 4), walls, 3))
+    for a, b, what in zip(*out, ("f", "den", "vel")):
+        np.testing.assert_array_equal(b, a, err_msg=what)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "fp16", "fp32_storage"])
+@pytest.mark.parametrize("lat,bc,tile,walls,solid", [
+    ((9, 7, 63), (P, P, P, P, P, P), "16,3,4", 0, 0.3),
+    ((2, 1, 64), (P, P, P, P, W, W), "", 1, 0.1),       # one row, its own neighbour; the planes too
+    ((33, 18, 34), (P, P, W, S, S, W), "11,5,8", 0, 0.2),
+    ((7, 13, 150), (W, W, S, S, P, P), "", 2, 0.1),
+    ((21, 11, 16), (V, D, W, W, S, W), "16,5,20", 2, 0.1),
+    ((5, 3, 400), (P, P, P, P, P, P), "200,1,5", 0, 0.97),  # rows and planes without a fluid site
+])
+def test_sparse_pairs_equal_single_steps(lat, bc, tile, walls, solid, precision, monkeypatch):
+    """The same in the sparse layout, from a few solid cells to nearly all,
+    against the rows layout's single steps."""
+    out = []
+    for pair in ("0", "1"):
+        monkeypatch.setenv("LB_PAIR", pair)
+        if tile:
+            monkeypatch.setenv("LB_PAIR_TILE", tile)
+        print(f"sparse pairs {pair}: {lat} {bc} tile {tile or 'auto'} walls {walls} {precision}", flush=True)
+        out.append(_run(lat, bc, precision, 1, (2, 7, 1, 4), walls, 3, "sparse" if pair == "1" else "rows", solid))
     for a, b, what in zip(*out, ("f", "den", "vel")):
         np.testing.assert_array_equal(b, a, err_msg=what)
