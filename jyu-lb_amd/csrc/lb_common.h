@@ -200,17 +200,19 @@ struct StepParams {
     const uint32_t* special;
     uint32_t nspecial, nzh;
     void* rec;  // if set: (rho, u*) of this step, 4 rows of the compute type (adjoint recompute):
-                // nq values by cell in the dense layouts, ps by compact site in the sparse layout
+                // nq values by cell in the dense layouts, nfp by compact site in the sparse layout
     // sparse layout (LB_LAYOUT_SPARSE), null otherwise: compact index of every
     // site (fluid sites only), site of every compact index, and the odd-step
-    // location of link l of compact site n at tab[link_slot(l) * ps + n]
+    // location of link l of compact site n at tab[link_slot(l) * nfp + n]
     const uint32_t* cidx;
     const uint32_t* site;
     const uint32_t* tab;
-    const uint32_t* tabc;   // compact form of tab (see step_sparse): SP_WORDS rows of ps words
-    const uint8_t* tabb;    // ... and its row of ps bytes (link slots 16 and 17), after them
+    const uint32_t* tabc;   // compact form of tab (see step_sparse): SP_WORDS rows of nfp words
+    const uint8_t* tabb;    // ... and its row of nfp bytes (link slots 16 and 17), after them
     const uint32_t* tabw;   // its base and alternate locations, SP_WAVE_WORDS per wave of 64 compact sites
     uint32_t nf;  // fluid sites = compact sites the step processes
+    uint32_t nfp;  // nf rounded up to 64: row stride of tab, tabc, tabb and rec
+    uint32_t bsh, bmul;  // blocks of the population array: see sp_elem
     // dissipation objective (k_diss): per site 19 population seeds, 3
     // acceleration seeds and the site's Pi^neq:Pi^neq, each an nq-long row of
     // the compute type; dscale = 1 / (fluid sites)
@@ -218,10 +220,22 @@ struct StepParams {
     double dscale;
 };
 
+// Sparse layout: compact site n keeps population l at sp_elem(n) + l*ps. The
+// array is in blocks of ps = 2^bsh sites, each with its 19 rows of ps values
+// (bmul = 18*ps), or one block of nfp sites (bsh 31, bmul 0). In one block
+// the 19 populations of a site lie in 19 regions far apart, and every wave's
+// loads and stores in as many pages; a block of 2^12 sites is 0.6 MB in FP64
+// (figures at sparse_blocks). Waves of 64 consecutive sites share a block.
+LBD uint32_t sp_elem(uint32_t n, uint32_t bsh, uint32_t bmul) { return n + (n >> bsh) * bmul; }
+// ... for a wave of consecutive sites: sp_elem(n) - n
+LBD uint32_t sp_base(const StepParams& p, uint32_t n) {
+    return (__builtin_amdgcn_readfirstlane(n) >> p.bsh) * p.bmul;
+}
+
 // expanded index of padded site c in the population array: population l of
 // site (i,j,k) lives at (i*ny + j)*rs + k + l*ps
 LBD int64_t eidx(const StepParams& p, uint32_t c) {
-    if (p.cidx) return p.cidx[c];  // sparse: population l of site c at cidx[c] + l*ps
+    if (p.cidx) return sp_elem(p.cidx[c], p.bsh, p.bmul);
     if (p.rs == p.d.nzp) return c;
     const uint32_t row = c / (uint32_t)p.d.nzp;
     return (int64_t)row * p.rs + (c - row * (uint32_t)p.d.nzp);

@@ -774,7 +774,7 @@ struct lb_solver {
     uint32_t nspecial = 0, special_cap = 0;
     uint32_t nzh = 0;  // Zou-He sites at the head of the special list
     // sparse layout: compact index per site, site per compact index, odd-step
-    // table; nfp = fluid sites rounded up to 64 (the population stride)
+    // table; nfp = fluid sites rounded up to 64 (the tables' row stride)
     bool sparse = false;
     int layout = LB_LAYOUT_AUTO;  // resolved at lb_create, or for LB_LAYOUT_AUTO at the first lb_finalize
     uint32_t* cidx = nullptr;
@@ -794,6 +794,8 @@ struct lb_solver {
     bool keep_prev = false, prev_valid = false;
     uint64_t sp_kinds[4] = {0, 0, 0, 0};  // link codes by kind (lb_sparse_codes)
     uint32_t nfp = 0;
+    uint32_t bsh = 31;  // blocks of the population array (sp_elem)
+    int sp_block = -1;  // LB_SP_BLOCK: log2 of a block's sites (6 or more), -1 by sparse_blocks
     uint8_t* phase = nullptr;
     double* den = nullptr;
     double* vel = nullptr;
@@ -950,6 +952,9 @@ static StepParams params(const lb_solver* s) {
         p.tabb = (const uint8_t*)(s->tabc + (size_t)SP_WORDS * s->nfp);
         p.tabw = s->tabw;
         p.nf = (uint32_t)s->nfluid;
+        p.nfp = s->nfp;
+        p.bsh = s->bsh;
+        p.bmul = s->bsh < 31 ? 18u << s->bsh : 0u;
     }
     return p;
 }
@@ -1193,7 +1198,8 @@ __global__ void k_compact(const uint32_t* mask, uint32_t nq, const uint32_t* wof
 // dense SoA view (element l*nq + c), in which odd_loc resolves bounce-back,
 // periodic, symmetric and z-wrapped links; a location on a non-fluid site
 // (which the link mask rules out) raises *err instead of being stored.
-__global__ void k_sparse_tab(StepParams q, const uint32_t* cidx, uint32_t nfp, uint32_t* tab, unsigned int* err) {
+__global__ void k_sparse_tab(StepParams q, const uint32_t* cidx, uint32_t nfp, uint32_t ps, uint32_t* tab,
+                             unsigned int* err) {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= q.nq) return;
     const uint32_t m = q.mask[c];
@@ -1208,9 +1214,9 @@ __global__ void k_sparse_tab(StepParams q, const uint32_t* cidx, uint32_t nfp, u
         const uint32_t ns = (ls >= 0 && ls < Q && cs >= 0 && cs < q.nq) ? cidx[cs] : ~0u;
         if (ns == ~0u) {
             atomicOr(err, 1u);
-            tab[(int64_t)link_slot(l) * nfp + n] = (uint32_t)REST * nfp + n;  // a valid location
+            tab[(int64_t)link_slot(l) * nfp + n] = (uint32_t)REST * ps + sp_elem(n, q.bsh, q.bmul);  // a valid location
         } else {
-            tab[(int64_t)link_slot(l) * nfp + n] = (uint32_t)ls * nfp + ns;
+            tab[(int64_t)link_slot(l) * nfp + n] = (uint32_t)ls * ps + sp_elem(ns, q.bsh, q.bmul);
         }
     }
 }
@@ -1237,8 +1243,9 @@ static bool sp_pull_on(const lb_solver* s, size_t array_bytes) {
 // alternate is the location of the lowest lane outside it, and every lane
 // with that location takes SP_ALT.
 // Counts of the link codes go to kinds[0..3]: near, SP_ALT, SP_BOUNCE, SP_FAR.
-__global__ __launch_bounds__(64) void k_sparse_pack(const uint32_t* tab, uint32_t nfp, uint32_t nf, uint32_t* tabc,
-                                                    uint32_t* tabw, unsigned long long* kinds) {
+__global__ __launch_bounds__(64) void k_sparse_pack(const uint32_t* tab, uint32_t nfp, uint32_t nf, uint32_t ps,
+                                                    uint32_t bsh, uint32_t bmul, uint32_t* tabc, uint32_t* tabw,
+                                                    unsigned long long* kinds) {
     const uint32_t w = blockIdx.x, lane = threadIdx.x;
     const uint32_t n = w * 64 + lane;  // < nfp: the grid is nfp / 64 waves
     const bool live = n < nf;
@@ -1247,7 +1254,7 @@ __global__ __launch_bounds__(64) void k_sparse_pack(const uint32_t* tab, uint32_
         if (l == REST) continue;
         const uint32_t sl = link_slot(l);
         const uint32_t loc = tab[(size_t)sl * nfp + n];
-        const bool bounce = live && loc == (uint32_t)l * nfp + n;
+        const bool bounce = live && loc == (uint32_t)l * ps + sp_elem(n, bsh, bmul);
         const bool cand = live && !bounce;
         const uint32_t d = loc - lane;
         const uint64_t cands = __ballot(cand);
@@ -1486,6 +1493,7 @@ static void layout_defaults(lb_solver* s, int layout) {
     if (const char* env = getenv("LB_EVEN_RR")) s->even_rr = strtol(env, nullptr, 10) != 0;
     s->sp_pull = -1;  // decided by sp_pull_on at lb_finalize
     if (const char* env = getenv("LB_SP_PULL")) s->sp_pull = strtol(env, nullptr, 10) != 0 ? 1 : 0;
+    if (const char* env = getenv("LB_SP_BLOCK")) s->sp_block = (int)std::min(std::max(strtol(env, nullptr, 10), 6l), 31l);  // 64 sites or more
     s->adj_pull = -1;
     s->pair = -1;
     if (const char* env = getenv("LB_PAIR")) s->pair = strtol(env, nullptr, 10) != 0 ? 1 : 0;
@@ -1536,11 +1544,11 @@ static void layout_defaults(lb_solver* s, int layout) {
 // In the sparse layout (nfluid is set) pairs are a candidate, which tune_pair
 // times: solid cells are columns that idle, every first step looks its
 // upstream sites up, and small lattices wait for that chain. Measured (ms per
-// step, single / paired): random spheres of 20% solid FP64 384x192x192 0.643 /
-// 0.492, 192^3 0.320 / 0.256, 128^3 0.0848 / 0.0803, 64^3 0.0149 / 0.0150;
-// FP32 256x128x128 0.0898 / 0.0896, 64^3 0.0085 / 0.0123; 40% solid FP64
-// 256^3 0.578 / 0.641. FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 /
-// 0.561) stay single.
+// step, single / paired): random spheres of 20% solid FP64 384x192x192 0.589 /
+// 0.483, 256x128x128 0.165 / 0.147, 320^3 1.383 / 1.167, 64^3 0.0149 / 0.0150;
+// FP32 384x192x192 0.303 / 0.289, 64^3 0.0085 / 0.0123; 40% solid FP64 256^3
+// 0.528 / 0.541. FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 / 0.561)
+// stay single.
 static bool pair_wanted(const lb_solver* s) {
     if (s->sp_pull >= 0 || s->pair == 0) return false;
     if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
@@ -1561,7 +1569,10 @@ static bool pair_wanted(const lb_solver* s) {
 // turn: 256^3 FP64 0.593 ms per step at 32x13x32 (predicted best), 0.642 at
 // 16x26x32, 0.681 at 64x5x32; 512x128x128 FP32 0.191 at 64x8x64 (predicted
 // best), 0.204 at 32x16x64; 48^3 FP64 0.0085 at 24x6x3 (predicted best),
-// 0.0096 at 48x8x2.
+// 0.0096 at 48x8x2. In the sparse layout the tiles' rows share lines with
+// their neighbours', which L2 joins while the neighbours keep step; long sweeps
+// drift apart (320^3 FP64 of 20% solid in tiles of 40x10: 1.136 ms per step in
+// chunks of 20 planes, 1.168 of 40, 1.258 of 80, 1.46 of 320).
 static void pair_tiling(lb_solver* s) {
     const Dims& d = s->d;
     const int NT = pair_threads(s->prec);
@@ -1589,7 +1600,8 @@ static void pair_tiling(lb_solver* s) {
         q.total = (uint32_t)total;
         const double lines = 1.0 + 1.3 * per_line / EK;  // lines read over lines needed
         const double iter = 1.3 + 4.6 * cols / NT * (0.5 + 0.5 * lines / 1.6);
-        const double t = (double)((total + cus - 1) / cus) * (chunk + 3) * iter;
+        const double drift = s->sparse ? 1.0 + 0.004 * std::min(chunk, 120) : 1.0;
+        const double t = (double)((total + cus - 1) / cus) * (chunk + 3) * iter * drift;
         if (!best.total || t < tbest) {
             best = q;
             tbest = t;
@@ -1862,41 +1874,58 @@ int lb_set_face_data(lb_solver* s, int face, const double* den_face, const doubl
     return LB_OK;
 }
 
+// log2 of the sites in a block of the sparse population array (sp_elem), or 31:
+// one block. Measured on random spheres of 20% solid (ms per step, one block /
+// blocks of 2^12 sites): single steps FP64 384x192x192 0.666 / 0.589, 320^3
+// 1.501 / 1.383, 128x64x64 0.0261 / 0.0252, FP32 384x192x192 0.331 / 0.303,
+// 128x64x64 0.0138 / 0.0133, FP16 320^3 0.440 / 0.425; paired FP64 384x192x192
+// 0.524 / 0.497. Smaller blocks put more waves across a boundary, where the
+// codes run out (2^10: 0.596), larger ones spread again (2^14: 0.606, 2^16:
+// 0.622). Small lattices lose by the boundaries (24x24x100 0.0063 / 0.0067).
+static uint32_t sparse_blocks(const lb_solver* s, uint64_t nfp) {
+    const uint32_t b = s->sp_block >= 0 ? (uint32_t)s->sp_block : nfp >= (1u << 18) ? 12 : 31;
+    // the padding of the last block does not refuse what one block can hold
+    return b < 31 && Q * ((((nfp - 1) >> b) + 1) << b) < (1ull << 32) ? b : 31;
+}
+
 // Sparse layout: compact the fluid sites in ascending dense order, size the
-// population array to them (stride nfp) and tabulate every odd-step location.
+// population array to them and tabulate every odd-step location.
 static int build_sparse(lb_solver* s) {
     const uint64_t nf = (uint64_t)s->nfluid;
     const uint64_t nfp = std::max<uint64_t>(64, (nf + 63) / 64 * 64);
-    if ((uint64_t)Q * nfp >= (1ull << 32))
+    const uint32_t bsh = sparse_blocks(s, nfp);
+    const uint64_t ps = bsh < 31 ? 1ull << bsh : nfp, fsize = Q * ((nfp + ps - 1) / ps * ps);
+    if (fsize >= (1ull << 32))
         return fail(LB_EINVAL, "sparse layout: %llu fluid sites exceed its 32-bit location table",
                     (unsigned long long)nf);
     const size_t ts = ts_size(s->prec);
     int rc;
     if (s->nfp != nfp) {
         const size_t o = s->nfp;
-        dfree(s, &s->f, Q * o * ts);
-        dfree(s, &s->snap, Q * o * ts);
+        dfree(s, &s->f, (size_t)s->fsize * ts);
+        dfree(s, &s->snap, (size_t)s->fsize * ts);
         dfree(s, (void**)&s->site, o * 4);
         dfree(s, (void**)&s->tab, (Q - 1) * o * 4);
         dfree(s, (void**)&s->tabc, SP_CODE_BYTES * o);
         dfree(s, (void**)&s->tabw, SP_WAVE_WORDS * (o / 64) * 4);
-        dfree(s, &s->f2, Q * o * ts);
+        dfree(s, &s->f2, (size_t)s->fsize * ts);
         s->nfp = 0;
-        if ((rc = dalloc(s, &s->f, Q * nfp * ts)) || (rc = dalloc(s, (void**)&s->site, nfp * 4)) ||
+        if ((rc = dalloc(s, &s->f, fsize * ts)) || (rc = dalloc(s, (void**)&s->site, nfp * 4)) ||
             (rc = dalloc(s, (void**)&s->tab, (Q - 1) * nfp * 4)) ||
             (rc = dalloc(s, (void**)&s->tabc, SP_CODE_BYTES * nfp)) ||
             (rc = dalloc(s, (void**)&s->tabw, SP_WAVE_WORDS * (nfp / 64) * 4)))
             return rc;
-        if (sp_pull_on(s, Q * nfp * ts)) dalloc_optional(s, &s->f2, Q * nfp * ts);
+        if (sp_pull_on(s, fsize * ts)) dalloc_optional(s, &s->f2, fsize * ts);
         s->pull_active = s->f2 != nullptr;
         s->nfp = (uint32_t)nfp;
     }
     if (!s->cidx && (rc = dalloc(s, (void**)&s->cidx, (size_t)s->nq * 4))) return rc;
-    s->ps = (int64_t)nfp;
+    s->bsh = bsh;
+    s->ps = (int64_t)ps;
     s->rs = 0;
-    s->fsize = (int64_t)Q * nfp;
-    HIPCHK(hipMemsetAsync(s->f, 0, Q * nfp * ts, s->stream));  // padding sites stay zero
-    if (s->f2) HIPCHK(hipMemsetAsync(s->f2, 0, Q * nfp * ts, s->stream));
+    s->fsize = (int64_t)fsize;
+    HIPCHK(hipMemsetAsync(s->f, 0, fsize * ts, s->stream));  // padding sites stay zero
+    if (s->f2) HIPCHK(hipMemsetAsync(s->f2, 0, fsize * ts, s->stream));
     HIPCHK(hipMemsetAsync(s->site, 0, nfp * 4, s->stream));
     // fluid sites per wave -> exclusive scan on the host -> compact indices
     const uint32_t nw = s->nq / 64;
@@ -1930,7 +1959,7 @@ static int build_sparse(lb_solver* s) {
     q.ps = s->nq;
     unsigned int* err = (unsigned int*)s->red;
     HIPCHK(hipMemsetAsync(err, 0, 4, s->stream));
-    k_sparse_tab<<<blocks_for(s->nq, 256), 256, 0, s->stream>>>(q, s->cidx, (uint32_t)nfp, s->tab, err);
+    k_sparse_tab<<<blocks_for(s->nq, 256), 256, 0, s->stream>>>(q, s->cidx, (uint32_t)nfp, (uint32_t)ps, s->tab, err);
     HIPCHK(hipGetLastError());
     unsigned int herr = 0;
     HIPCHK(hipMemcpyAsync(&herr, err, 4, hipMemcpyDeviceToHost, s->stream));
@@ -1938,8 +1967,8 @@ static int build_sparse(lb_solver* s) {
     if (herr) return fail(LB_EHIP, "sparse layout set-up: a link resolves to a non-fluid site");
     unsigned long long* kinds = (unsigned long long*)s->red;
     HIPCHK(hipMemsetAsync(kinds, 0, sizeof(s->sp_kinds), s->stream));
-    k_sparse_pack<<<(unsigned)(nfp / 64), 64, 0, s->stream>>>(s->tab, (uint32_t)nfp, (uint32_t)nf, s->tabc,
-                                                             s->tabw, kinds);
+    k_sparse_pack<<<(unsigned)(nfp / 64), 64, 0, s->stream>>>(s->tab, (uint32_t)nfp, (uint32_t)nf, (uint32_t)ps, q.bsh,
+                                                             q.bmul, s->tabc, s->tabw, kinds);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(s->sp_kinds, kinds, sizeof(s->sp_kinds), hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));

@@ -353,8 +353,8 @@ __global__ __launch_bounds__(TILE) void k_diss_special(StepParams p) {
 // ---------------------------------------------------------------------------
 // Compact site n (fluid sites in ascending dense order, so consecutive threads
 // mostly hold consecutive k of one lattice row) keeps population l at
-// f[l*ps + n]. An even step reads and writes only these slots. An odd step
-// reads link l from tab[link_slot(l)*ps + n], the element that the dense
+// f[sp_elem(n) + l*ps]. An even step reads and writes only these slots. An odd
+// step reads link l from tab[link_slot(l)*nfp + n], the element that the dense
 // resolver (odd_loc) names for it, mapped to compact indices at
 // lb_finalize: upstream slot, own slot for bounce-back, or the periodic /
 // mirrored source; it writes f*_opp(l) back there. FULL sites may carry
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(TILE) void k_diss_special(StepParams p) {
 // periodic face at the end of a row); SP_BOUNCE, the own slot l; SP_FAR, a
 // location read from the 32-bit table (0.2% of the links on a random-sphere
 // medium). A site's 18 codes are two 32-bit words of eight links and a byte
-// of two, in two rows of ps words and a row of ps bytes: three loads per
+// of two, in two rows of nfp words and a row of nfp bytes: three loads per
 // wave, 9 bytes per site (5-bit codes in three words, 12 bytes, measured
 // 0.7% slower in FP64 and 2% in FP32; 8-bit codes, 18 bytes, slower still).
 
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(TILE) void k_diss_special(StepParams p) {
 // this can be in flight together; the rare SP_FAR links are fixed up in one
 // wave-uniform branch.
 LBD void sparse_locs(const StepParams& p, const uint32_t n, uint32_t* loc) {
-    const uint32_t ps = (uint32_t)p.ps;
+    const uint32_t ps = (uint32_t)p.ps, e = sp_base(p, n) + n;
     const uint32_t* B = p.tabw + (size_t)__builtin_amdgcn_readfirstlane(n >> 6) * SP_WAVE_WORDS;
     uint32_t base[Q - 1], alt[Q - 1], w[SP_WORDS + 1];
 #pragma unroll
@@ -394,26 +394,26 @@ LBD void sparse_locs(const StepParams& p, const uint32_t n, uint32_t* loc) {
     // lines wait for the neighbouring waves (FP16 0.6% and FP32 about 1%
     // faster on the 768x384x384 medium, FP64 unchanged)
 #pragma unroll
-    for (int q = 0; q < SP_WORDS; ++q) w[q] = __builtin_nontemporal_load(p.tabc + (size_t)q * ps + n);
+    for (int q = 0; q < SP_WORDS; ++q) w[q] = __builtin_nontemporal_load(p.tabc + (size_t)q * p.nfp + n);
     w[SP_WORDS] = __builtin_nontemporal_load(p.tabb + n);
     const uint32_t lane = n & 63u;  // waves start at multiples of 64
     uint32_t far = 0;
 #pragma unroll
     for (int l = 0; l < Q; ++l) {
         if (l == REST) {
-            loc[l] = REST * ps + n;
+            loc[l] = REST * ps + e;
             continue;
         }
         const int sl = link_slot(l);
         const uint32_t code = sp_code(w, sl);
         const uint32_t near = base[sl] + lane + code;  // modulo 2^32: the base may be below 0
-        loc[l] = code < SP_ALT ? near : code == SP_ALT ? alt[sl] : (uint32_t)l * ps + n;
+        loc[l] = code < SP_ALT ? near : code == SP_ALT ? alt[sl] : (uint32_t)l * ps + e;
         far |= (code == SP_FAR ? 1u : 0u) << sl;
     }
     if (__ballot(far != 0)) {
 #pragma unroll
         for (int l = 0; l < Q; ++l)
-            if (l != REST && ((far >> link_slot(l)) & 1u)) loc[l] = p.tab[link_slot(l) * ps + n];
+            if (l != REST && ((far >> link_slot(l)) & 1u)) loc[l] = p.tab[link_slot(l) * p.nfp + n];
     }
 }
 
@@ -425,7 +425,8 @@ LBD void step_sparse_at(const StepParams& p, const uint32_t n, const uint32_t* l
     using TC = typename Var<P>::TC;
     constexpr bool SH = Var<P>::SH;
     TS* F = (TS*)p.f;
-    const uint32_t ps = (uint32_t)p.ps;  // 19 * ps < 2^32 (lb_finalize)
+    const uint32_t ps = (uint32_t)p.ps;  // the array has fewer than 2^32 elements (lb_finalize)
+    const uint32_t wb = sp_base(p, n), nfp = p.nfp;
     const TC* A = (const TC*)p.acc;
     const bool need_c = FULL || DISS || A || p.store_dv;  // uniform
     const uint32_t c = need_c ? p.site[n] : 0u;
@@ -435,7 +436,7 @@ LBD void step_sparse_at(const StepParams& p, const uint32_t n, const uint32_t* l
 
     // population l of this site: a wave-uniform base plus the 32-bit lane
     // offset n (n * sizeof(TS) < 2^32)
-    auto own = [&](int l) { return uniform_ptr(F + (int64_t)l * ps) + n; };
+    auto own = [&](int l) { return uniform_ptr(F + (wb + (uint32_t)l * ps)) + n; };
     TC f[Q];
     if constexpr (!ODD) {
 #pragma unroll
@@ -471,12 +472,12 @@ LBD void step_sparse_at(const StepParams& p, const uint32_t n, const uint32_t* l
     } else if (FULL && p.moving && (m & M_MOVING)) {
         p.den[c] = SH ? p.rho0 + (double)ds : (double)den;
     }
-    if (p.rec) {  // by compact site: rows of ps values
+    if (p.rec) {  // by compact site: rows of nfp values
         TC* R = (TC*)p.rec;
         R[n] = den;
-        R[ps + n] = vel[0];
-        R[2 * ps + n] = vel[1];
-        R[3 * ps + n] = vel[2];
+        R[nfp + n] = vel[0];
+        R[2 * nfp + n] = vel[1];
+        R[3 * nfp + n] = vel[2];
     }
     if constexpr (!ODD) {
 #pragma unroll
@@ -484,7 +485,7 @@ LBD void step_sparse_at(const StepParams& p, const uint32_t n, const uint32_t* l
     } else if constexpr (PULL) {
         TS* G = (TS*)p.f2;
 #pragma unroll
-        for (int l = 0; l < Q; ++l) stf<P, NTSE>(uniform_ptr(G + (int64_t)opp(l) * ps) + n, f[l], p.scale);
+        for (int l = 0; l < Q; ++l) stf<P, NTSE>(uniform_ptr(G + (wb + (uint32_t)opp(l) * ps)) + n, f[l], p.scale);
     } else {
 #pragma unroll
         for (int l = 0; l < Q; ++l) stf<P, NTSO>(l == REST ? own(l) : F + loc[l], f[opp(l)], p.scale);
@@ -557,7 +558,7 @@ namespace lb {
 // lam: cotangents of the post-collision populations; mu: of the streamed ones.
 // c: the site's cell (read only for a per-site acceleration field and the
 // dissipation seeds); r: its index in the record and in x.gacc, rows of rs
-// values (the cell and nq in the dense layouts, the compact site and ps in
+// values (the cell and nq in the dense layouts, the compact site and nfp in
 // the sparse layout).
 template <int P, int RLX>
 LBD void adj_core(const StepParams& p, const AdjParams& x, const uint32_t c, const uint32_t r, const int64_t rs,
@@ -716,7 +717,7 @@ __global__ __launch_bounds__(TILE) void k_adj_sp(StepParams p, AdjParams x) {
     const uint32_t n = tile * p.tile + threadIdx.x;
     if (n >= p.nf) return;
     TC* L = (TC*)x.lam;
-    const uint32_t ps = (uint32_t)p.ps;
+    const uint32_t ps = (uint32_t)p.ps, wb = sp_base(p, n);
     const uint32_t c = ZH || x.seed || p.acc ? p.site[n] : 0u;  // uniform choice
     const uint32_t m = ZH ? p.mask[c] : M_FLUID;
     int i = 0, j = 0, k = 0;
@@ -730,13 +731,13 @@ __global__ __launch_bounds__(TILE) void k_adj_sp(StepParams p, AdjParams x) {
         for (int l = 0; l < Q; ++l) lam[opp(l)] = L[loc[l]];
     } else {
 #pragma unroll
-        for (int l = 0; l < Q; ++l) lam[l] = ld_stream<NTE>(uniform_ptr(L + (int64_t)opp(l) * ps) + n);
+        for (int l = 0; l < Q; ++l) lam[l] = ld_stream<NTE>(uniform_ptr(L + (wb + (uint32_t)opp(l) * ps)) + n);
     }
-    adj_core<P, RLX>(p, x, c, n, ps, m, ZH && (m & M_ZH_ANY) != 0, i, j, k, lam, mu);
+    adj_core<P, RLX>(p, x, c, n, p.nfp, m, ZH && (m & M_ZH_ANY) != 0, i, j, k, lam, mu);
 #pragma unroll
     for (int l = 0; l < Q; ++l) {
         if constexpr (ODD) L[loc[l]] = mu[l];
-        else st_stream<NTE>(uniform_ptr(L + (int64_t)l * ps) + n, mu[l]);
+        else st_stream<NTE>(uniform_ptr(L + (wb + (uint32_t)l * ps)) + n, mu[l]);
     }
 }
 
@@ -760,7 +761,7 @@ __global__ __launch_bounds__(TILE) void k_adj_sp_pull(StepParams p, AdjParams x)
     if (n >= p.nf) return;
     const TC* L = (const TC*)x.lam;
     TC* L2 = (TC*)x.lam2;
-    const uint32_t ps = (uint32_t)p.ps;
+    const uint32_t ps = (uint32_t)p.ps, wb = sp_base(p, n);
     const uint32_t c = ZH || x.seed || p.acc ? p.site[n] : 0u;  // uniform choice
     const uint32_t m = ZH ? p.mask[c] : M_FLUID;
     int i = 0, j = 0, k = 0;
@@ -771,9 +772,9 @@ __global__ __launch_bounds__(TILE) void k_adj_sp_pull(StepParams p, AdjParams x)
     sparse_locs(p, n, loc);
 #pragma unroll
     for (int l = 0; l < Q; ++l) lam[opp(l)] = L[loc[l]];
-    adj_core<P, RLX>(p, x, c, n, ps, m, ZH && (m & M_ZH_ANY) != 0, i, j, k, lam, mu);
+    adj_core<P, RLX>(p, x, c, n, p.nfp, m, ZH && (m & M_ZH_ANY) != 0, i, j, k, lam, mu);
 #pragma unroll
-    for (int l = 0; l < Q; ++l) st_stream<NTE>(uniform_ptr(L2 + (int64_t)l * ps) + n, mu[l]);
+    for (int l = 0; l < Q; ++l) st_stream<NTE>(uniform_ptr(L2 + (wb + (uint32_t)l * ps)) + n, mu[l]);
 }
 
 
@@ -881,7 +882,7 @@ __global__ void k_post_f(StepParams p, int next_odd, double* out) {
             int64_t loc;
             if (next_odd) loc = e + (int64_t)lo * p.ps;
             else if (!p.tab) loc = odd_loc(p, m, e, lo, i, j, k);
-            else loc = lo == REST ? e + (int64_t)REST * p.ps : p.tab[(int64_t)link_slot(lo) * p.ps + e];
+            else loc = lo == REST ? e + (int64_t)REST * p.ps : p.tab[(int64_t)link_slot(lo) * p.nfp + p.cidx[c]];
             v = (double)ldf<P, false>(F + loc, p.inv_scale);
             if (Var<P>::SH) v += (l == REST ? 12.0 / 36.0 : nnz(l) == 1 ? 2.0 / 36.0 : 1.0 / 36.0) * p.rho0;
         }
@@ -940,7 +941,7 @@ template <int P, int RLX>
 static void launch_adj(const StepParams& ps, const AdjParams& x, bool odd, hipStream_t st) {
     StepParams p = ps;  // the adjoint kernels run TILE threads per workgroup
     p.tile = TILE;
-    p.ntiles = ((p.tab ? (uint32_t)p.ps : p.nq) + TILE - 1) / TILE;
+    p.ntiles = ((p.tab ? p.nfp : p.nq) + TILE - 1) / TILE;
     const unsigned grid = tile_grid(p);
     if (p.tab) {  // sparse layout
         if (x.lam2) {  // pull form, the same kernel at either parity

@@ -36,7 +36,7 @@
 // four planes, each loaded an iteration ahead. Tiles' rows start and end
 // anywhere in a line: L2 joins the stores (1.80 GB written for 1.72 GB of
 // populations on 384x192x192 cells of 20% solid). ms per step there, single /
-// paired: FP64 0.643 / 0.492; 256x128x128 0.179 / 0.154.
+// paired: FP64 0.589 / 0.483; 256x128x128 0.165 / 0.147.
 #pragma once
 #include <type_traits>
 
@@ -214,10 +214,10 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         }
     };
     // The same in the sparse layout: the compact indices of the planes around
-    // are in LDS (a ring of four planes, I0 the plane before). 32-bit element
-    // offsets reach the whole array (19 * ps < 2^32).
+    // are in LDS as sp_elem gives them (a ring of four planes, I0 the plane
+    // before). 32-bit element offsets reach the whole array (lb_finalize).
     const int EX = EK + 2, xc = (jj + 1) * EX + kk + 1;
-    uint32_t nN = 0, nA = 0, nB = 0;  // own compact index in planes i + 1, i, i - 1
+    uint32_t nN = 0, nA = 0, nB = 0;  // own sp_elem in planes i + 1, i, i - 1
     auto gather_sp = [&](auto part, const uint32_t* I0, const uint32_t* I1, const uint32_t* I2, uint32_t m) {
         constexpr int PT = decltype(part)::value;
         if (!(m & M_FLUID)) return;
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
     };
     auto keep_idx = [&](int slot) {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) idx[slot * NC + e * NT + t] = cv[e];
+        for (int e = 0; e < 2; ++e) idx[slot * NC + e * NT + t] = sp_elem(cv[e], p.bsh, p.bmul);
     };
     // One collision, on the streamed populations f of the site (ip, jw, kw).
     // What is loaded in a branch is waited for there: a wait behind it would
@@ -461,17 +461,27 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         arrive();
         asm volatile("" : "+v"(mNN));
         if (second) {
-            char* G = (char*)p.f2 + (SP ? 0 : (int64_t)ipB * plane);
-            uint64_t step = (uint64_t)psb;
-            uint32_t o = SP ? nB * (uint32_t)sizeof(TS) : own;
-            asm volatile("" : "+s"(step), "+v"(o));  // not multiplied out, nor widened, ahead of the loop
             // Plain stores: L2 joins the lines that two tiles share. With
             // non-temporal ones 256^3 FP64 ran 0.615 ms per step (plain
             // 0.572) and tiles that split lines 0.968 (33x12x32; 0.751).
+            uint64_t step = (uint64_t)psb;
+            if constexpr (SP) {
+                uint64_t a = (uint64_t)((TS*)p.f2 + nB);
+                asm volatile("" : "+s"(step), "+v"(a));
 #pragma unroll
-            for (int sl = 0; sl < Q; ++sl) {
-                *(TS*)(uniform_ptr(G) + o) = to_ts<P>(h[opp(sl)], p.scale);
-                G += step;
+                for (int sl = 0; sl < Q; ++sl) {
+                    *(__attribute__((address_space(1))) TS*)a = to_ts<P>(h[opp(sl)], p.scale);
+                    a += step;
+                }
+            } else {
+                char* G = (char*)p.f2 + (int64_t)ipB * plane;
+                uint32_t o = own;
+                asm volatile("" : "+s"(step), "+v"(o));  // not multiplied out, nor widened, ahead of the loop
+#pragma unroll
+                for (int sl = 0; sl < Q; ++sl) {
+                    *(TS*)(uniform_ptr(G) + o) = to_ts<P>(h[opp(sl)], p.scale);
+                    G += step;
+                }
             }
         }
         r0 = s9;

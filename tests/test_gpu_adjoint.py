@@ -395,6 +395,24 @@ def test_adjoint_identical_in_sparse_layout(precision, rlx, steps_bc):
     np.testing.assert_array_equal(out[1][2], out[0][2])
 
 
+@pytest.mark.parametrize("pull", ["0", "1"], ids=["in_place", "pull"])
+def test_adjoint_identical_in_sparse_blocks(pull, monkeypatch):
+    """The cotangents, checkpoints and records of a population array in blocks
+    of 64 sites: objective and both gradients as in the dense layout."""
+    out = []
+    for layout in ("rows", "sparse"):
+        if layout == "sparse":
+            monkeypatch.setenv("LB_SP_BLOCK", "6")
+            monkeypatch.setenv("LB_ADJ_PULL", pull)
+        s, prof, amp = make_channel(TRT, "fp64", steps_bc=(WALL, SYMMETRIC), seed=8, layout=layout)
+        acc, fden, fvel, g = _inputs(s)
+        s.engine.snapshot()
+        out.append(_adjoint(s, acc, fden, fvel, g, 30, 7))
+    assert out[0][0] == out[1][0]
+    np.testing.assert_array_equal(out[1][1], out[0][1])
+    np.testing.assert_array_equal(out[1][2], out[0][2])
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("pre_steps", [0, 1], ids=["from_odd", "from_even"])
 @pytest.mark.parametrize("layout", ["sparse", "rows"])

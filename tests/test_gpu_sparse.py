@@ -150,6 +150,25 @@ def test_sparse_pull_steps_on_reference_scenarios(name, monkeypatch):
         np.testing.assert_array_equal(b[k], a[k], err_msg=f"{name} {k}")
 
 
+@pytest.mark.parametrize("block", ["6", "8"])
+@pytest.mark.parametrize("steps", ["in_place", "pull", "pairs"])
+@pytest.mark.parametrize("name", NAMES)
+def test_sparse_blocks_on_reference_scenarios(name, steps, block, monkeypatch):
+    """The population array in blocks (from 2^18 fluid sites on; here of 64 and
+    256 sites, so that waves cross their boundaries in every link) against the
+    rows layout, FP64, bit for bit, in each kind of step."""
+    a = _run_fixture(name, layout="rows")
+    monkeypatch.setenv("LB_SP_BLOCK", block)
+    if steps == "pairs":
+        monkeypatch.setenv("LB_PAIR", "1")
+    else:
+        monkeypatch.setenv("LB_SP_PULL", "1" if steps == "pull" else "0")
+    print(f"blocks of 2^{block} sites, {steps}, scenario {name}", flush=True)
+    b = _run_fixture(name, layout="sparse")
+    for k in a:
+        np.testing.assert_array_equal(b[k], a[k], err_msg=f"{name} {k}")
+
+
 def test_sparse_porous_medium_matches_oracle():
     import jyulb_oracle as jo
     from jyulb.isothermal import Solver
