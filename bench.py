@@ -4,9 +4,9 @@ Headline workload: the porous medium of 768 x 384 x 384 cells (113M cells,
 90.6M fluid sites): seeded random spheres of radius 6..12 up to 20 % solid
 (jyulb.geometry.porous_spheres, seed 5), D3Q19 TRT (magic 3/16), tau = 0.6,
 gravity gx = 1e-6, periodic on every face. A "step" is one fused
-stream+collide pass over the lattice (an AA step in place, or a pull step into
-the second population array), with the populations resident in HBM, timed with
-HIP events on the stream the kernels run on. `value` is FP64 MLUPS
+stream+collide of every fluid site (in a pass of its own, in place or into the
+second population array, or in a pass that does two), with the populations
+resident in HBM, timed with HIP events on the stream the kernels run on. `value` is FP64 MLUPS
 (fluid-site updates) in the Solver's default layout ("auto", which picks the
 sparse fluid-only layout for this medium); FP32 on shifted populations, FP16
 storage / FP32 arithmetic and FP32 storage / FP64 arithmetic are in
@@ -45,16 +45,24 @@ C5_NAME = ("porous medium 768x384x384 (113M cells; spheres r 6..12, 20% solid, s
            "(magic 3/16), tau=0.6, gx=1e-6, periodic")
 
 
-def step_kernel(prec, layout, rlx="1", pull=False):
-    """rocprof name pattern of the bulk step kernel (both parities; with the
-    sparse layout's pull steps, the one kernel of every step after the
-    first of a call)."""
+def step_kernel(prec, layout, rlx="1", pull=False, pair=False):
+    """rocprof name pattern of the bulk step kernel: that of two steps at once
+    where they are paired, else of single steps (both parities; with pull
+    steps, the one kernel of every step after the first of a call)."""
     p = {"fp64": 0, "fp32": 1, "fp16": 2, "fp32_storage": 3}[prec]
+    if pair:
+        return f"k_pair<{p},{rlx},*>"
     if layout == "sparse":
         return f"k_step_sp_pull<{p},{rlx},false>" if pull else f"k_step_sp<{p},{rlx},*,false>"
     if prec == "fp16" and rlx == "1":
         return "k_step_h<1,true,true>" if pull else "k_step_h<1,*>"
     return f"k_step<{p},{rlx},true,true>" if pull else f"k_step<{p},{rlx},*>"
+
+
+def bytes_per_site(prec, pair):
+    """What a site's step has to move: its populations in and out, once per
+    step, or once per two where steps are paired."""
+    return BYTES_PER_SITE[prec] // (2 if pair else 1)
 
 
 # ---------------------------------------------------------------------------
@@ -208,11 +216,13 @@ def headline(precs, steps, warmup, layout, solid):
               file=sys.stderr, flush=True)
         t, wall = time_device(s, steps, warmup)
         fields[prec] = s.engine.download_den_vel()[1]
-        gbs = BYTES_PER_SITE[prec] * nfl * steps / t / 1e9
+        pair = s.engine.paired_steps()
+        gbs = bytes_per_site(prec, pair) * nfl * steps / t / 1e9
         res[prec] = dict(mlups=round(nfl * steps / t / 1e6, 1), mlups_cells=round(ncell * steps / t / 1e6, 1),
                          ms_per_step=round(1e3 * t / steps, 5), achieved_gbs=round(gbs, 1),
                          frac=round(gbs / PEAK_HBM_GBS, 4), layout=lay,
-                         kernel=step_kernel(prec, lay, pull=s.engine.pull_steps()), pull=s.engine.pull_steps(),
+                         kernel=step_kernel(prec, lay, pull=s.engine.pull_steps(), pair=pair),
+                         pull=s.engine.pull_steps(), pair=pair,
                          nfluid=nfl, device_bytes=int(s.engine.info()["device_bytes"]),
                          fp16_scale=s.engine.info()["fp16_scale"])
         if lay == "sparse":
@@ -243,10 +253,12 @@ def cavity_workload(n, steps, warmup, precs):
         s, nfl = make_cavity(n, prec)
         t, _ = time_device(s, steps, max(warmup, 60))
         lay = s.engine.layout()
-        gbs = BYTES_PER_SITE[prec] * nfl * steps / t / 1e9
+        pair = s.engine.paired_steps()
+        gbs = bytes_per_site(prec, pair) * nfl * steps / t / 1e9
         out[prec] = dict(mlups=round(nfl * steps / t / 1e6, 1), ms_per_step=round(1e3 * t / steps, 5),
                          achieved_gbs=round(gbs, 1), frac=round(gbs / PEAK_HBM_GBS, 4), layout=lay,
-                         kernel=step_kernel(prec, lay, pull=s.engine.pull_steps()), pull=s.engine.pull_steps())
+                         kernel=step_kernel(prec, lay, pull=s.engine.pull_steps(), pair=pair),
+                         pull=s.engine.pull_steps(), pair=pair)
         print(f"[bench] cavity {n}^3 {prec} {lay}: {out[prec]['mlups']} MLUPS", file=sys.stderr, flush=True)
         del s
         torch.cuda.synchronize()
@@ -492,7 +504,7 @@ def main():
                    "fluid_sites": m["nfluid"], "layout": m["layout"], "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": m["achieved_gbs"], "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": m["frac"], "traffic": load_traffic(main_p, m["layout"]), "kernel": m["kernel"],
-                     "bytes_per_site": BYTES_PER_SITE[main_p], "copy_ceiling_gbs": ceiling,
+                     "bytes_per_site": bytes_per_site(main_p, m["pair"]), "copy_ceiling_gbs": ceiling,
                      "frac_of_copy": m["frac_of_copy"]},
         "variants": res,
         "precision_error_vs_fp64": errors,

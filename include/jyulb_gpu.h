@@ -110,24 +110,25 @@ int lb_set_face_data(lb_solver *s, int face, const double *den_face, const doubl
 int lb_finalize(lb_solver *s, int64_t *nfluid);
 
 /* The step loop of Solver.evolve (isothermal.pyx:1408-1415): `steps` fused
- * AA stream+collide steps. den/vel of the fluid sites are stored on the last
- * step. Asynchronous on the handle's stream, except that the FP16 storage
- * variant checks its stored magnitudes (and rescales them by a power of two)
+ * stream+collide steps. den/vel of the fluid sites are stored on the last
+ * step. Asynchronous on the handle's stream, except that the first long call
+ * may time launches on its own steps, and that the FP16 storage variant checks its stored magnitudes (and rescales them by a power of two)
  * at the start and every 64 steps (LB_FP16_CHECK), failing with LB_ESTATE if
  * a population overflowed. A recorded adjoint forward pass no longer applies
  * afterwards (see lb_adj_backward). */
 int lb_evolve(lb_solver *s, uint32_t steps);
 
-/* Pinned host memory (hipHostMalloc) for the Solver's own arrays, so that
- * the copies of lb_evolve_host run at full DMA speed; lb_host_free releases
- * it. */
+/* Pinned host memory (hipHostMalloc) for the Solver's own arrays, which the
+ * kernels of lb_evolve_host then read and write in place; lb_host_free
+ * releases it. */
 int lb_host_alloc(size_t bytes, void **ptr);
 int lb_host_free(void *ptr);
 
 /* The Solver's halo-padded host fields (isothermal.pyx:243-248): phase u8
  * [NI][NJ][NK], den f64 [NI][NJ][NK], vel and acc f64 [NI][NJ][NK][3] with
  * NI = nx + 2, NJ = ny + 2, NK = nz + 2. lb_evolve_host reads and writes them
- * in place. Any host memory works; lb_host_alloc memory is faster. They must
+ * in place. Any host memory works; memory of lb_host_alloc is read and written
+ * by kernels over the bus, other memory through staged copies. They must
  * stay valid while bound; four NULLs unbind them. Allocates a device copy of
  * the four fields. */
 int lb_bind_host_fields(lb_solver *s, uint8_t *phase, double *den, double *vel, double *acc);
@@ -290,6 +291,14 @@ int lb_sparse_codes(lb_solver *s, uint64_t counts[4]);
  * FP32 storage; LB_SP_PULL=0/1 in the environment decides instead, also for
  * the dense layouts. Results are identical either way. */
 int lb_pull_steps(lb_solver *s, int *on);
+
+/* Whether lb_evolve takes two steps per pass over the populations (no
+ * counterpart in the reference) where a call has two left: into a second
+ * population array, allocated by the first such call; without the memory for
+ * it steps stay single. Where it depends on the flow, the first call that is
+ * long enough times both, and *on is 0 until then. LB_PAIR=0/1 in the
+ * environment decides instead. Results are identical either way. */
+int lb_paired_steps(lb_solver *s, int *on);
 
 /* The population layout in use (LB_LAYOUT_*; LB_LAYOUT_AUTO until the first
  * lb_finalize resolves it). */

@@ -1541,20 +1541,22 @@ static void layout_defaults(lb_solver* s, int layout) {
 // where three planes of populations exceed the kernel's 32-bit offsets, nor
 // where LB_SP_PULL asks for single steps of one kind. rs and ps are set.
 //
-// In the sparse layout (nfluid is set) pairs are a candidate, which tune_pair
-// times: solid cells are columns that idle, every first step looks its
-// upstream sites up, and small lattices wait for that chain. Measured (ms per
-// step, single / paired): random spheres of 20% solid FP64 384x192x192 0.589 /
-// 0.483, 256x128x128 0.165 / 0.147, 320^3 1.383 / 1.167, 64^3 0.0149 / 0.0150;
-// FP32 384x192x192 0.303 / 0.289, 64^3 0.0085 / 0.0123; 40% solid FP64 256^3
-// 0.528 / 0.541. FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 / 0.561)
-// stay single.
+// In the sparse layout (nfluid is set) solid cells are columns that idle, every
+// first step looks its upstream sites up, and small lattices wait for that
+// chain. Measured (ms per step, single / paired): random spheres of 20% solid
+// FP64 384x192x192 0.589 / 0.483, 256x128x128 0.165 / 0.147, 320^3 1.383 /
+// 1.167, 64^3 0.0149 / 0.0150; FP32 384x192x192 0.303 / 0.289, 256x128x128
+// 0.085 / 0.088; 40% solid FP64 256^3 0.528 / 0.541. FP64 takes them; so does FP32
+// from 2^23 sites (768x384x384 2.57 / 2.28), which below lets tune_pair time
+// both; FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 /
+// 0.561) stay single.
 static bool pair_wanted(const lb_solver* s) {
     if (s->sp_pull >= 0 || s->pair == 0) return false;
     if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
-    if (s->sparse)
-        return s->pair > 0 || (s->autotune && (s->prec == LB_FP64 || s->prec == LB_FP32_SHIFTED) &&
-                               s->nfluid >= (1 << 19) && s->nfluid * 10 >= s->ncell * 7);
+    if (s->sparse) {
+        const bool prec = s->prec == LB_FP64 || (s->prec == LB_FP32_SHIFTED && (s->autotune || s->nfluid >= (1 << 23)));
+        return s->pair > 0 || (prec && s->nfluid >= (1 << 19) && s->nfluid * 10 >= s->ncell * 7);
+    }
     const uint64_t ts = ts_size(s->prec);
     return 3 * (uint64_t)s->d.ny * (uint64_t)s->rs * ts + Q * (uint64_t)s->ps * ts < (1ull << 32);
 }
@@ -1566,9 +1568,9 @@ static bool pair_wanted(const lb_solver* s) {
 // column shortens (two barriers, LDS, a collision's chain) and one by the
 // column, which the lines its row reads raise: 34 doubles span 3.4 lines of
 // 128 bytes on average, 66 span 5.4. Measured with every tiling forced in
-// turn: 256^3 FP64 0.593 ms per step at 32x13x32 (predicted best), 0.642 at
-// 16x26x32, 0.681 at 64x5x32; 512x128x128 FP32 0.191 at 64x8x64 (predicted
-// best), 0.204 at 32x16x64; 48^3 FP64 0.0085 at 24x6x3 (predicted best),
+// turn: 256^3 FP64 0.567 ms per step at 32x13x32 (predicted best), 0.668 at
+// 64x5x32; 512x128x128 FP32 0.191 at 64x8x64 (predicted best), 0.204 at
+// 32x16x64; 48^3 FP64 0.0085 at 24x6x3 (predicted best),
 // 0.0096 at 48x8x2. In the sparse layout the tiles' rows share lines with
 // their neighbours', which L2 joins while the neighbours keep step; long sweeps
 // drift apart (320^3 FP64 of 20% solid in tiles of 40x10: 1.136 ms per step in
@@ -1628,7 +1630,7 @@ static void pair_tiling(lb_solver* s) {
             const int TK = (d.nz + ntk - 1) / ntk, TK8 = (TK + 7) / 8 * 8;
             if (TK > NT / 3) continue;
             if (ntk > 1 && TK < 20) break;
-            all_of(ntk > 1 && !s->sparse ? TK8 : TK);  // tiles start on half a line at least: unaligned ones (37x11x86) ran 256^3 FP64 at 0.886
+            all_of(ntk > 1 && !s->sparse ? TK8 : TK);  // tiles start on half a line at least: unaligned ones (37x11x86) ran 256^3 FP64 at 0.702
         }
     }
     memcpy(best.wall, s->pq.wall, sizeof(best.wall));
@@ -2006,13 +2008,14 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
     if (s->pair_on) {
         // Pairs are faster where walls stand still and values have 4 bytes or
         // more (ms per step, single / paired: 256^3 channel FP64 0.894 /
-        // 0.593, FP32 0.451 / 0.323; 160^3 FP32 0.121 / 0.119; 48^3 FP64
-        // 0.0215 / 0.0085). With moving walls or FP16 storage, where the
-        // collisions bind, it depends: cavities 256^3 FP64 0.928 / 0.648, FP16
-        // 0.284 / 0.389, 160^3 FP32 0.118 / 0.132, 64^3 FP64 0.0164 / 0.0171,
-        // 48^3 FP64 0.0128 / 0.0102; 64^3 channel FP16 0.0184 / 0.0112.
-        // In the sparse layout it depends on the solid too, whose columns idle.
-        s->pair_tune = s->pair < 0 && s->autotune && (s->moving || s->sparse || s->prec == LB_FP16_STORAGE);
+        // 0.567, FP32 0.451 / 0.300; 48^3 FP64 0.0215 / 0.0085). With moving
+        // walls or FP16 storage, where the collisions bind, it depends:
+        // cavities 256^3 FP64 0.928 / 0.624, FP32 0.501 / 0.343, FP16 0.284 /
+        // 0.389, 64^3 FP64 0.0164 / 0.0171, 48^3 FP64 0.0128 / 0.0102; 64^3
+        // channel FP16 0.0184 / 0.0112. Sparse FP32: see pair_wanted.
+        s->pair_tune = s->pair < 0 && s->autotune &&
+                       (s->moving || s->prec == LB_FP16_STORAGE ||
+                        (s->sparse && s->prec != LB_FP64 && s->nfluid < (1 << 23)));
         if (s->pair_tune) s->pair_on = false;
         else s->tune = false;  // few single steps are left to tune
     }
@@ -2126,9 +2129,6 @@ static int fp16_guard(lb_solver* s) {
     return LB_OK;
 }
 
-// `n` steps with the solver's current launch configuration; the last one
-// stores den/vel if `store_last`. FP16 storage runs its guard every
-// f16_check steps.
 // One step from the state in s->f, whose parity is `odd` (updated). Where
 // pull steps are active and the second array is there, an odd step is a pull
 // step: it leaves the state an even step leaves, in s->f2, which then becomes
@@ -2177,6 +2177,9 @@ static void swap_rho(PairParams& q) {
     q.rho_in = in;
 }
 
+// `n` steps with the solver's current launch configuration, two at a time where
+// they are paired; the last one stores den/vel if `store_last`. FP16 storage
+// runs its guard every f16_check steps.
 static int run_steps(lb_solver* s, uint32_t n, bool store_last) {
     StepParams p = params(s);
     PairParams q = s->pq;
@@ -3199,6 +3202,12 @@ int lb_sparse_codes(lb_solver* s, uint64_t* counts) {
     if (!s->finalized || s->layout != LB_LAYOUT_SPARSE)
         return fail(LB_ESTATE, "lb_sparse_codes needs a finalized solver in the sparse layout");
     for (int k = 0; k < 4; ++k) counts[k] = s->sp_kinds[k];
+    return LB_OK;
+}
+
+int lb_paired_steps(lb_solver* s, int* on) {
+    if (!s || !on) return fail(LB_EINVAL, "null argument");
+    *on = s->pair_on && !(s->moving && !s->mov_pairs) ? 1 : 0;
     return LB_OK;
 }
 

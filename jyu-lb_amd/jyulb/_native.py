@@ -95,6 +95,7 @@ def lib():
                      ctypes.POINTER(ctypes.c_uint64), dp], ctypes.c_int),
         "lb_sparse_codes": ([H, ctypes.POINTER(ctypes.c_uint64)], ctypes.c_int),
         "lb_pull_steps": ([H, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
+        "lb_paired_steps": ([H, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "lb_synchronize": ([H], ctypes.c_int),
         "lb_set_face_data_device": ([H, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p], ctypes.c_int),
         "lb_objective": ([H, ctypes.c_int, ctypes.c_int, dp], ctypes.c_int),
@@ -343,6 +344,13 @@ class Engine:
         """True when the solver steps by pull steps (a second population array)."""
         v = ctypes.c_int()
         self.call("lb_pull_steps", ctypes.byref(v))
+        return bool(v.value)
+
+    def paired_steps(self):
+        """True when evolve takes two steps per pass over the populations (once
+        a long call has timed it, where it depends on the flow)."""
+        v = ctypes.c_int()
+        self.call("lb_paired_steps", ctypes.byref(v))
         return bool(v.value)
 
     def layout(self):
