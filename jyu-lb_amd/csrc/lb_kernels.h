@@ -828,8 +828,11 @@ LBD void comp_der_vel(const Dims& d, const double* vel, uint32_t nq, uint32_t m,
 
 // Solver._init_f, isothermal.pyx:1028-1105: f1 = P(heq + (1-omega)(-2 tau/3) rho S),
 // written as the state after an even AA step (f*_l in slot opp(l)).
+// Bound by the 90 velocities it gathers per site: with 256 VGPRs (2 waves per
+// SIMD) 3.3 ms at 256^3 FP64; held to 128, which spilled 628 bytes per lane,
+// 6.6 ms, to 168 5.3 ms, and with one wave per SIMD 3.3 ms.
 template <int P>
-__global__ void k_init(StepParams p) {
+__global__ __launch_bounds__(256, 2) void k_init(StepParams p) {
     using TS = typename Var<P>::TS;
     constexpr bool SH = Var<P>::SH;
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
