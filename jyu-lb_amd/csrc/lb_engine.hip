@@ -1223,12 +1223,11 @@ __global__ void k_sparse_tab(StepParams q, const uint32_t* cidx, uint32_t nfp, u
 
 // Whether the sparse layout steps by pull steps (run_steps), given the bytes
 // of one population array. Pull steps against odd AA steps in place (ms per
-// step, sparse porous media of 20% solid): FP64 0.0295 / 0.0254 at
-// 128x64x64, 0.197 / 0.186 at 256x128x128, 0.650 / 0.686 at 384x192x192,
-// 1.545 / 1.587 at 512x256x256, 5.28 / 5.46 at 768x384x384; FP32 2.76 /
-// 2.83 and FP32 storage 2.77 / 2.80 at 768x384x384, within 1% either way
-// from 384x192x192 to 512x256x256; FP16 1.59 / 1.57 at 768x384x384. Below
-// about 1 GiB of populations the lattice sits largely in the 256 MiB last-level
+// step, sparse porous media of 20% solid): FP64 0.0276 / 0.0256 at
+// 128x64x64, 0.176 / 0.169 at 256x128x128, 0.584 / 0.597 at 384x192x192,
+// 1.379 / 1.424 at 320^3; FP32 0.704 / 0.719 and FP32 storage 0.734 / 0.742
+// at 320^3; FP16 0.443 / 0.417 there. Below about 1 GiB of populations the
+// lattice sits largely in the 256 MiB last-level
 // cache and the even AA step's purely local access wins; FP16 keeps the AA
 // steps (and half the population memory).
 static bool sp_pull_on(const lb_solver* s, size_t array_bytes) {
