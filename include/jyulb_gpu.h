@@ -112,10 +112,14 @@ int lb_finalize(lb_solver *s, int64_t *nfluid);
 /* The step loop of Solver.evolve (isothermal.pyx:1408-1415): `steps` fused
  * stream+collide steps. den/vel of the fluid sites are stored on the last
  * step. Asynchronous on the handle's stream, except that the first long call
- * may time launches on its own steps, and that the FP16 storage variant checks its stored magnitudes (and rescales them by a power of two)
- * at the start and every 64 steps (LB_FP16_CHECK), failing with LB_ESTATE if
- * a population overflowed. A recorded adjoint forward pass no longer applies
- * afterwards (see lb_adj_backward). */
+ * may time launches on its own steps, and that the FP16 storage variant checks
+ * its stored magnitudes (and rescales them by a power of two) at the start and
+ * every 64 steps (LB_FP16_CHECK), failing with LB_ESTATE if a population
+ * overflowed. A recorded adjoint forward pass no longer applies afterwards
+ * (see lb_adj_backward). A call whose steps are captured into a graph keeps
+ * all later steps of the handle single (lb_paired_steps), so that replays and
+ * plain calls step the same array: each with an even number of steps between
+ * two replays, none of them counted for a replay (lb_info). */
 int lb_evolve(lb_solver *s, uint32_t steps);
 
 /* Pinned host memory (hipHostMalloc) for the Solver's own arrays, which the

@@ -765,6 +765,7 @@ struct lb_solver {
     int pair = -1;
     bool pair_on = false;
     bool pair_tune = false;  // ... to be settled by timing both (tune_pair), with single steps until then
+    bool captured = false;   // steps were captured into a graph: no pairs from then on (pairs_barred)
     int pair_tile[3] = {0, 0, 0};  // LB_PAIR_TILE: inner columns along k and j, planes (0: pair_tiling chooses)
     PairParams pq{};
     void* f = nullptr;
@@ -1556,7 +1557,7 @@ static void layout_defaults(lb_solver* s, int layout) {
 // both; FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 /
 // 0.561) stay single.
 static bool pair_wanted(const lb_solver* s) {
-    if (s->sp_pull >= 0 || s->pair == 0) return false;
+    if (s->sp_pull >= 0 || s->pair == 0 || s->captured) return false;
     if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
     if (s->sparse) {
         const bool prec = s->prec == LB_FP64 || (s->prec == LB_FP32_SHIFTED && (s->autotune || s->nfluid >= (1 << 23)));
@@ -2151,22 +2152,33 @@ static void one_step(lb_solver* s, StepParams& p, int& odd) {
     }
 }
 
-static bool capturing(const lb_solver* s) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s->stream, &capture) != hipSuccess) {
+// Whether this call's steps have to stay single. A captured graph replays with
+// the arrays that its steps were captured with, while a pair leaves the state
+// in the other array: a pair between two replays would have the next replay
+// advance an old state. So steps under capture are single, and so are all of
+// this handle's later ones, in the array that the graph holds; the second
+// array goes back at the first call outside a capture.
+static bool pairs_barred(lb_solver* s) {
+    hipStreamCaptureStatus now = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s->stream, &now) != hipSuccess) {
         (void)hipGetLastError();
-        return true;
+        return true;  // this call only
     }
-    return capture != hipStreamCaptureStatusNone;
+    if (now != hipStreamCaptureStatusNone) {
+        s->captured = true;
+    } else if (s->captured && (s->pair_on || s->pair_tune)) {
+        s->pair_on = s->pair_tune = false;
+        if (!s->tune) drop_pull_candidate(s);
+    }
+    return s->captured;
 }
 
 // Whether this call's steps may be paired: the second population array is
 // there (the first such call allocates it; without the memory, steps stay
-// single) and the stream is not being captured, as a graph replays with the
-// arrays it was captured with, while pairs swap them.
+// single).
 static bool pairs_ready(lb_solver* s) {
     if (!s->pair_on || (s->moving && !s->mov_pairs)) return false;
-    if (capturing(s)) return false;
+    if (pairs_barred(s)) return false;
     if (s->f2) return true;
     const size_t fb = (size_t)s->fsize * ts_size(s->prec);
     dalloc_optional(s, &s->f2, fb);
@@ -2293,6 +2305,10 @@ static int tune_candidates(const lb_solver* s, StepCfg* c) {
 constexpr int TUNE_PULL_STEPS = 2 * TUNE_STEPS + 1;
 static int tune_pull(lb_solver* s) {
     if (!s->f2 || s->pull_active) return LB_OK;
+    if (s->captured) {  // pull steps leave the state in the other array too (pairs_barred)
+        drop_pull_candidate(s);
+        return LB_OK;
+    }
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool ok = true;
     for (hipEvent_t& e : ev) ok = ok && hipEventCreate(&e) == hipSuccess;
@@ -2444,6 +2460,7 @@ static int capture_prev(lb_solver* s) {
 // first long call, then the steps (den/vel stored on the last one).
 static int evolve_steps(lb_solver* s, uint32_t steps) {
     int rc = LB_OK;
+    const bool barred = pairs_barred(s);
     if (s->prec == LB_FP16_STORAGE && (s->f16_dirty || s->f16_since >= s->f16_check) && (rc = fp16_guard(s)))
         return rc;
     if (s->tune) {
@@ -2460,7 +2477,7 @@ static int evolve_steps(lb_solver* s, uint32_t steps) {
             steps -= (uint32_t)(s->steps - before);
         }
     }
-    if (s->pair_tune && !s->tune && steps > (uint32_t)PAIR_TUNE_STEPS && !capturing(s)) {
+    if (s->pair_tune && !s->tune && steps > (uint32_t)PAIR_TUNE_STEPS && !barred) {
         const uint64_t before = s->steps;
         if ((rc = tune_pair(s))) return rc;
         steps -= (uint32_t)(s->steps - before);
@@ -3212,7 +3229,7 @@ int lb_sparse_codes(lb_solver* s, uint64_t* counts) {
 
 int lb_paired_steps(lb_solver* s, int* on) {
     if (!s || !on) return fail(LB_EINVAL, "null argument");
-    *on = s->pair_on && !(s->moving && !s->mov_pairs) ? 1 : 0;
+    *on = s->pair_on && !s->captured && !(s->moving && !s->mov_pairs) ? 1 : 0;
     return LB_OK;
 }
 
