@@ -1116,9 +1116,9 @@ __global__ void k_ladd_prep(const uint32_t* mask, const double* vel, Dims d, uin
 }
 
 // The paired steps' form of the moving sites (PairParams::mov): site q's
-// moving links, and its wall velocity among the n in walls. *first becomes the
-// lowest q whose velocity is not among them, or 0 where one site's walls
-// differ (*split).
+// moving links, and its wall velocity among the n in walls, into word unless
+// that is null. *first becomes the lowest q whose velocity is not among them;
+// *split is set where one site's walls differ.
 struct Walls {
     double v[PAIR_WALLS][3];
     int n;
@@ -1157,7 +1157,7 @@ __global__ void k_pair_walls(const uint32_t* mask, const double* vel, Dims d, ui
     int e = 0;
     while (e < walls.n && !same_bits(v, walls.v[e])) ++e;
     if (e == walls.n) atomicMin(first, q);
-    else word[cell[q]] = links | (uint32_t)e << 18;
+    else if (word) word[cell[q]] = links | (uint32_t)e << 18;
 }
 __global__ void k_wall_of(const uint32_t* mask, const double* vel, Dims d, uint32_t nq, const uint32_t* cell,
                           const unsigned int* q, double* v) {
@@ -1298,38 +1298,56 @@ __global__ __launch_bounds__(64) void k_sparse_pack(const uint32_t* tab, uint32_
     ((uint8_t*)(tabc + (size_t)SP_WORDS * nfp))[n] = (uint8_t)word[SP_WORDS];
 }
 
+// The arrays of pair_walls, 12 bytes per cell: held only where pairs use them.
+static void drop_pair_walls(lb_solver* s) {
+    s->mov_pairs = false;
+    dfree(s, (void**)&s->mov_word, (size_t)s->nq * 4);
+    dfree(s, (void**)&s->den2, (size_t)s->nq * 8);
+}
+
 // Whether the paired steps can take this lattice's moving walls (mov_pairs),
-// and their form of them: every site's moving walls share one velocity, and
-// there are at most PAIR_WALLS of those (a lid, two sliding plates). Each
-// round finds one more velocity. Other walls keep single steps, which read 18
-// sums per site: in the paired steps those loads wait behind the next plane's
-// (256^3 cavity, FP64: 0.713 ms per step with the sums loaded, 0.648 so; 48^3
-// 0.0128 and 0.0102).
+// and their form of them: every site's moving walls share one velocity, there
+// are at most PAIR_WALLS of those (a lid, two sliding plates), and there is
+// memory for the form. Each round finds one more velocity. Other walls keep
+// single steps, which read 18 sums per site: in the paired steps those loads
+// wait behind the next plane's (256^3 cavity, FP64: 0.713 ms per step with the
+// sums loaded, 0.648 so; 48^3 0.0128 and 0.0102).
 static int pair_walls(lb_solver* s) {
     s->mov_pairs = false;
-    int rc;
-    if (!s->mov_word && (rc = dalloc(s, (void**)&s->mov_word, (size_t)s->nq * 4))) return rc;
-    if (!s->den2 && (rc = dalloc(s, (void**)&s->den2, (size_t)s->nq * 8))) return rc;
     Walls walls;
     memset(&walls, 0, sizeof(walls));
     unsigned int* first = (unsigned int*)s->red;  // first, split; the velocity after them
     double* v = s->red + 1;
+    auto sites = [&](uint32_t* word) {
+        k_pair_walls<<<blocks_for(s->nmov, 256), 256, 0, s->stream>>>(s->mask, s->vel, s->d, s->nq, s->mov_cell, s->nmov,
+                                                                      walls, word, first, first + 1);
+    };
     for (;; ++walls.n) {
         const unsigned int init[2] = {~0u, 0u};
         unsigned int got[2];
         HIPCHK(hipMemcpyAsync(first, init, sizeof(init), hipMemcpyHostToDevice, s->stream));
-        k_pair_walls<<<blocks_for(s->nmov, 256), 256, 0, s->stream>>>(s->mask, s->vel, s->d, s->nq, s->mov_cell, s->nmov,
-                                                                      walls, s->mov_word, first, first + 1);
+        sites(nullptr);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(got, first, sizeof(got), hipMemcpyDeviceToHost, s->stream));
         HIPCHK(hipStreamSynchronize(s->stream));
-        if (got[1] || (got[0] != ~0u && walls.n == PAIR_WALLS)) return LB_OK;
+        if (got[1] || (got[0] != ~0u && walls.n == PAIR_WALLS)) {
+            drop_pair_walls(s);
+            return LB_OK;
+        }
         if (got[0] == ~0u) break;
         k_wall_of<<<1, 1, 0, s->stream>>>(s->mask, s->vel, s->d, s->nq, s->mov_cell, first, v);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(walls.v[walls.n], v, 24, hipMemcpyDeviceToHost, s->stream));
         HIPCHK(hipStreamSynchronize(s->stream));
     }
+    if (!s->mov_word) dalloc_optional(s, (void**)&s->mov_word, (size_t)s->nq * 4);
+    if (!s->den2) dalloc_optional(s, (void**)&s->den2, (size_t)s->nq * 8);
+    if (!s->mov_word || !s->den2) {
+        drop_pair_walls(s);
+        return LB_OK;
+    }
+    sites(s->mov_word);
+    HIPCHK(hipGetLastError());
     memcpy(s->pq.wall, walls.v, sizeof(walls.v));
     s->mov_pairs = true;
     return LB_OK;
@@ -1688,6 +1706,14 @@ static int layout_arrays(lb_solver* s, int layout) {
 // The second array of a dense pull-step candidate that was not chosen.
 static void drop_pull_candidate(lb_solver* s) {
     if (s->f2 && !s->pull_active && !s->pair_on && !s->pair_tune) dfree(s, &s->f2, (size_t)s->fsize * ts_size(s->prec));
+}
+
+// Single steps from here on: what the pairs held goes back (the second array
+// unless pull steps use it, or the launch tuner still has them to time).
+static void drop_pairs(lb_solver* s) {
+    s->pair_on = s->pair_tune = false;
+    drop_pair_walls(s);
+    if (!s->tune) drop_pull_candidate(s);
 }
 
 int lb_create(const lb_config* cfg, lb_solver** out) {
@@ -2167,8 +2193,7 @@ static bool pairs_barred(lb_solver* s) {
     if (now != hipStreamCaptureStatusNone) {
         s->captured = true;
     } else if (s->captured && (s->pair_on || s->pair_tune)) {
-        s->pair_on = s->pair_tune = false;
-        if (!s->tune) drop_pull_candidate(s);
+        drop_pairs(s);
     }
     return s->captured;
 }
@@ -2184,7 +2209,7 @@ static bool pairs_ready(lb_solver* s) {
     dalloc_optional(s, &s->f2, fb);
     if (s->f2 && s->prec == LB_FP16_STORAGE)  // the FP16 guard reads more than the fluid sites
         k_fill<uint64_t><<<(unsigned)((fb / 8 + 255) / 256), 256, 0, s->stream>>>((uint64_t*)s->f2, fb / 8, 0);
-    s->pair_on = s->f2 != nullptr;
+    if (!s->f2) drop_pairs(s);
     return s->pair_on;
 }
 
@@ -2430,7 +2455,7 @@ static int tune_pair(lb_solver* s) {
     if (s->tune_verbose)
         fprintf(stderr, "[jyulb] single steps %.4f ms, paired steps %.4f ms per step\n", ms[0] / PAIR_TUNE,
                 ms[1] / PAIR_TUNE);
-    drop_pull_candidate(s);
+    if (!s->pair_on) drop_pairs(s);
     return rc;
 }
 

@@ -1,0 +1,95 @@
+"""What the paired steps hold besides single steps' arrays, and that it goes
+back where they do not run."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+P, W = 1, 0
+LAT = (24, 12, 40)
+VELOCITIES = [(0.02, -0.01, 0.03), (0.0, 0.04, 0.0), (-0.03, 0.0, 0.01), (0.01, 0.01, -0.02), (0.0, -0.02, 0.02)]
+
+
+def _fields(plates, gap=3):
+    """Plates of 2 x 2 x 3 cells in a row along i, `gap` cells of fluid between
+    them (with one, the sites there reach two of them)."""
+    phase, vel = np.ones(LAT, dtype=np.uint8), np.zeros(LAT + (3,))
+    for b in range(plates):
+        at = (slice(1 + (2 + gap) * b, 3 + (2 + gap) * b), slice(3, 5), slice(4, 7))
+        phase[at] = 0
+        vel[at] = VELOCITIES[b]
+    return phase, vel
+
+
+def _engine(plates, layout="rows", precision="fp64", gap=3):
+    from jyulb import _native
+    e = _native.Engine(LAT, 1, 0.05, (1e-5, 0.0, 0.0), (P, P, W, W, P, P), precision=precision, layout=layout)
+    phase, vel = _fields(plates, gap)
+    e.upload_phase(phase)
+    e.upload_den_vel(np.ones(LAT), vel)
+    e.finalize()
+    return e
+
+
+def _bytes(e):
+    return e.info()["device_bytes"]
+
+
+@pytest.mark.parametrize("layout", ["rows", "sparse"])
+@pytest.mark.parametrize("plates,gap,pairs", [(4, 3, True), (5, 2, False), (2, 1, False)],
+                         ids=["four_velocities", "five_velocities", "two_at_one_site"])
+def test_walls_that_keep_single_steps_hold_nothing(plates, gap, pairs, layout, monkeypatch):
+    monkeypatch.setenv("LB_PAIR", "0")
+    single = _engine(plates, layout, gap=gap)
+    single.evolve(6)
+    monkeypatch.setenv("LB_PAIR", "1")
+    e = _engine(plates, layout, gap=gap)
+    e.evolve(6)
+    assert e.paired_steps() == pairs
+    assert (_bytes(e) > _bytes(single)) == pairs
+    np.testing.assert_array_equal(e.download_post_f(), single.download_post_f())
+
+
+def test_walls_that_come_to_differ_give_it_back(monkeypatch):
+    """Velocities that change between calls: one, then two at one site, then
+    one again."""
+    out = []
+    for pair in ("0", "1"):
+        monkeypatch.setenv("LB_PAIR", pair)
+        e = _engine(2, gap=1)
+        solid = _fields(2, gap=1)[0] == 0
+        for scale, pairs in ((0.0, True), (1.0, False), (0.0, True)):
+            vel = np.zeros(LAT + (3,))
+            vel[solid] = (0.01, 0.02, 0.0)
+            vel[4:][solid[4:]] *= 1.0 + scale  # the second plate's
+            e.upload_den_vel(np.ones(LAT), vel)
+            e.refresh_walls()
+            e.evolve(5)
+            if pair == "1":
+                assert e.paired_steps() == pairs
+            out.append(e.download_post_f())
+    for a, b in zip(out[:3], out[3:]):
+        np.testing.assert_array_equal(b, a)
+
+
+def test_capture_gives_it_back(monkeypatch):
+    import torch
+    monkeypatch.setenv("LB_PAIR", "0")
+    single = _engine(1)
+    monkeypatch.setenv("LB_PAIR", "1")
+    e = _engine(1)
+    st = torch.cuda.Stream()
+    e.set_stream(st.cuda_stream)
+    with torch.cuda.stream(st):
+        e.evolve(4)
+        torch.cuda.synchronize()
+        assert _bytes(e) > _bytes(single)
+        g = torch.cuda.CUDAGraph()
+        g.capture_begin()
+        e.evolve(2)
+        g.capture_end()
+        g.replay()
+        e.evolve(2)
+        torch.cuda.synchronize()
+    single.evolve(8)
+    assert _bytes(e) == _bytes(single)
+    np.testing.assert_array_equal(e.download_post_f(), single.download_post_f())
