@@ -30,6 +30,7 @@
 #include <math.h>
 #include <stdarg.h>
 #include <algorithm>
+#include <atomic>
 #include <utility>
 #include <vector>
 #include <stdio.h>
@@ -732,6 +733,8 @@ __global__ void k_face_bound(const double* fden, const double* fvel, size_t n, d
 // handle
 // ---------------------------------------------------------------------------
 struct lb_solver {
+    std::recursive_mutex mx;  // held by calls that use what pairs hold: another thread's call may want it back (make_room)
+    int device = 0;
     lb_config cfg;
     Dims d;
     int NI, NJ, NK;
@@ -830,7 +833,7 @@ struct lb_solver {
     int64_t nfluid = 0;
     uint64_t steps = 0;
     int next_odd = 1;
-    uint64_t bytes = 0;
+    std::atomic<uint64_t> bytes{0};
     // adjoint (checkpointed reverse pass)
     void* ckpt = nullptr;  // (nseg + 1) states: segment starts and the final state
     size_t ckpt_bytes = 0;
@@ -869,29 +872,57 @@ static size_t tc_size(int prec) { return prec == LB_FP64 || prec == LB_FP32_STOR
 static size_t rec_row(const lb_solver* s) { return s->sparse ? (size_t)s->nfp : (size_t)s->nq; }
 
 static void dfree(lb_solver* s, void** p, size_t n);
+static bool give_back(lb_solver* s);
 
-static int dalloc(lb_solver* s, void** p, size_t n) {
+// The handles there are, for make_room. Never destroyed: handles may outlive it.
+struct Handles {
+    std::mutex mx;
+    std::vector<lb_solver*> all;
+};
+static Handles& handles() {
+    static Handles* h = new Handles;
+    return *h;
+}
+
+// Room for an allocation of s that failed: what paired steps hold, which
+// single steps do without, is given back by s, and then by the device's other
+// handles that no call is using.
+static bool make_room(lb_solver* s) {
+    if (give_back(s)) return true;
+    bool any = false;
+    std::lock_guard<std::mutex> lock(handles().mx);
+    for (lb_solver* o : handles().all) {
+        if (o == s || o->device != s->device || !o->mx.try_lock()) continue;
+        any = give_back(o) || any;
+        o->mx.unlock();
+    }
+    return any;
+}
+
+static hipError_t malloc_or_room(lb_solver* s, void** p, size_t n) {
     hipError_t e = hipMalloc(p, n);
-    if (e != hipSuccess && s->f2 && (s->pair_on || s->pair_tune) && !s->pull_active) {
-        // the paired steps' second array makes room: single steps in place
+    while (e == hipErrorOutOfMemory && make_room(s)) {
         (void)hipGetLastError();
-        (void)hipStreamSynchronize(s->stream);
-        s->pair_on = s->pair_tune = false;
-        dfree(s, &s->f2, (size_t)s->fsize * ts_size(s->prec));
         e = hipMalloc(p, n);
     }
+    return e;
+}
+
+static int dalloc(lb_solver* s, void** p, size_t n) {
+    const hipError_t e = malloc_or_room(s, p, n);
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // or the thread's next launch check would report it
         return fail(LB_ENOMEM, "hipMalloc(%zu bytes) failed: %s", n, hipGetErrorString(e));
     }
     s->bytes += n;
     return LB_OK;
 }
 
-// An optional array (the second population or cotangent array of the pull
-// steps): null, and the steps run in place, if the device cannot hold it.
-static void dalloc_optional(lb_solver* s, void** p, size_t n) {
-    if (hipMalloc(p, n) != hipSuccess) {
+// An optional array: null, and the steps do without, if the device cannot hold
+// it. Those of the pull steps (room) come before what paired steps hold.
+static void dalloc_optional(lb_solver* s, void** p, size_t n, bool room = false) {
+    if ((room ? malloc_or_room(s, p, n) : hipMalloc(p, n)) != hipSuccess) {
         *p = nullptr;
         (void)hipGetLastError();
         return;
@@ -1695,7 +1726,7 @@ static int layout_arrays(lb_solver* s, int layout) {
     // launch tuner's last candidate (tune_step), which frees the second
     // array again if the in-place steps stay faster.
     if (s->sp_pull == 1 || (s->sp_pull < 0 && s->tune)) {
-        dalloc_optional(s, &s->f2, fb);
+        dalloc_optional(s, &s->f2, fb, true);
         if (s->f2) HIPCHK(hipMemset(s->f2, 0, fb));
         s->pull_active = s->f2 && s->sp_pull == 1;
     }
@@ -1708,12 +1739,32 @@ static void drop_pull_candidate(lb_solver* s) {
     if (s->f2 && !s->pull_active && !s->pair_on && !s->pair_tune) dfree(s, &s->f2, (size_t)s->fsize * ts_size(s->prec));
 }
 
+// Bytes that only paired steps use.
+static uint64_t pair_bytes(const lb_solver* s) {
+    uint64_t n = 0;
+    if (s->f2 && !s->pull_active && (s->pair_on || s->pair_tune)) n += (uint64_t)s->fsize * ts_size(s->prec);
+    if (s->mov_word) n += (uint64_t)s->nq * 4;
+    if (s->den2) n += (uint64_t)s->nq * 8;
+    return n;
+}
+
 // Single steps from here on: what the pairs held goes back (the second array
 // unless pull steps use it, or the launch tuner still has them to time).
 static void drop_pairs(lb_solver* s) {
     s->pair_on = s->pair_tune = false;
     drop_pair_walls(s);
     if (!s->tune) drop_pull_candidate(s);
+}
+
+static bool give_back(lb_solver* s) {
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
+    if (!pair_bytes(s)) return false;
+    (void)hipDeviceSynchronize();
+    const bool tune = s->tune;
+    s->tune = false;  // not kept as the launch tuner's candidate either
+    drop_pairs(s);
+    s->tune = tune;
+    return true;
 }
 
 int lb_create(const lb_config* cfg, lb_solver** out) {
@@ -1723,6 +1774,7 @@ int lb_create(const lb_config* cfg, lb_solver** out) {
     if (rc) return rc;
     if (lb_device_count() < 1) return fail(LB_EHIP, "no HIP device available");
     lb_solver* s = new lb_solver();
+    (void)hipGetDevice(&s->device);
     s->cfg = *cfg;
     s->d.nx = cfg->lat[0];
     s->d.ny = cfg->lat[1];
@@ -1804,12 +1856,21 @@ int lb_create(const lb_config* cfg, lb_solver** out) {
         lb_destroy(s);
         return fail(LB_EHIP, "device initialisation failed");
     }
+    {
+        std::lock_guard<std::mutex> lock(handles().mx);
+        handles().all.push_back(s);
+    }
     *out = s;
     return LB_OK;
 }
 
 int lb_destroy(lb_solver* s) {
     if (!s) return LB_OK;
+    {
+        std::lock_guard<std::mutex> lock(handles().mx);
+        auto& all = handles().all;
+        all.erase(std::remove(all.begin(), all.end(), s), all.end());
+    }
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     else (void)hipDeviceSynchronize();
     void* ptrs[] = {s->f,     s->mask, s->wclass, s->special, s->phase, s->den,  s->vel,  s->acc,
@@ -1949,7 +2010,7 @@ static int build_sparse(lb_solver* s) {
             (rc = dalloc(s, (void**)&s->tabc, SP_CODE_BYTES * nfp)) ||
             (rc = dalloc(s, (void**)&s->tabw, SP_WAVE_WORDS * (nfp / 64) * 4)))
             return rc;
-        if (sp_pull_on(s, fsize * ts)) dalloc_optional(s, &s->f2, fsize * ts);
+        if (sp_pull_on(s, fsize * ts)) dalloc_optional(s, &s->f2, fsize * ts, true);
         s->pull_active = s->f2 != nullptr;
         s->nfp = (uint32_t)nfp;
     }
@@ -2011,6 +2072,7 @@ static int build_sparse(lb_solver* s) {
 
 int lb_finalize(lb_solver* s, int64_t* nfluid) {
     if (!s) return fail(LB_EINVAL, "null handle");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
     inputs_changed(s);
     if (!s->phase_set) return fail(LB_ESTATE, "phase field not uploaded");
     s->finalized = false;  // until the populations below are initialised
@@ -2087,6 +2149,7 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
 
 int lb_refresh_walls(lb_solver* s) {
     if (!s) return fail(LB_EINVAL, "null handle");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
     inputs_changed(s);
     if (!s->phase_set) return fail(LB_ESTATE, "phase field not uploaded");
     int rc = build_mask(s, true);
@@ -2199,7 +2262,7 @@ static bool pairs_barred(lb_solver* s) {
 }
 
 // Whether this call's steps may be paired: the second population array is
-// there (the first such call allocates it; without the memory, steps stay
+// there (the first such call allocates it; without the room, steps stay
 // single).
 static bool pairs_ready(lb_solver* s) {
     if (!s->pair_on || (s->moving && !s->mov_pairs)) return false;
@@ -2519,6 +2582,7 @@ static int evolve_steps(lb_solver* s, uint32_t steps) {
 
 int lb_evolve(lb_solver* s, uint32_t steps) {
     if (!s) return fail(LB_EINVAL, "null handle");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
     if (!s->finalized) return fail(LB_ESTATE, "Finalize solver initialization before calling evolve");
     state_advanced(s);  // an earlier adjoint forward pass no longer applies
     if (s->nfluid < 1 || steps == 0) return LB_OK;
@@ -2663,6 +2727,7 @@ static int load_host_fields(lb_solver* s) {
 
 int lb_load_host_fields(lb_solver* s) {
     if (!s) return fail(LB_EINVAL, "null handle");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
     if (!s->finalized) return fail(LB_ESTATE, "solver not finalized");
     if (!s->h_phase) return fail(LB_ESTATE, "no host fields bound (lb_bind_host_fields)");
     inputs_changed(s);
@@ -2719,6 +2784,7 @@ static int evolve_pinned(lb_solver* s, uint32_t steps) {
 
 int lb_evolve_host(lb_solver* s, uint32_t steps) {
     if (!s) return fail(LB_EINVAL, "null handle");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
     if (!s->finalized) return fail(LB_ESTATE, "Finalize solver initialization before calling evolve");
     if (!s->h_phase) return fail(LB_ESTATE, "no host fields bound (lb_bind_host_fields)");
     inputs_changed(s);
@@ -2976,6 +3042,7 @@ int lb_adj_forward(lb_solver* s, uint32_t steps, uint32_t interval, int face, in
     const bool diss = face == LB_OBJ_DISSIPATION;
     if (!s || !J || face < 0 || face > LB_OBJ_DISSIPATION || (!diss && (axis < 0 || axis > 2)))
         return fail(LB_EINVAL, "invalid argument");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
     if (!s->finalized) return fail(LB_ESTATE, "solver not finalized");
     if (steps < 1 || interval < 1) return fail(LB_EINVAL, "steps and checkpoint interval must be >= 1");
     if (s->prec != LB_FP64 && s->prec != LB_FP32_SHIFTED)
@@ -3063,6 +3130,7 @@ int lb_adj_forward(lb_solver* s, uint32_t steps, uint32_t interval, int face, in
 
 static int adj_backward(lb_solver* s, int gface_id, double* grad_acc, double* grad_face, bool device) {
     if (!s) return fail(LB_EINVAL, "null handle");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
     if (!s->adj_ready)
         return fail(LB_ESTATE, "lb_adj_backward needs the lb_adj_forward pass of the current state and inputs: "
                     "an evolve step, an input upload or a restore since the forward pass invalidates it");
@@ -3083,7 +3151,7 @@ static int adj_backward(lb_solver* s, int gface_id, double* grad_acc, double* gr
     // (22.5 against 24.3 us per adjoint step).
     const size_t lbytes = (size_t)s->fsize * tcs;
     const bool want_lpull = s->adj_pull >= 0 ? s->adj_pull != 0 : lbytes >= ((size_t)1 << 30);
-    if (want_lpull && !s->lam2) dalloc_optional(s, &s->lam2, lbytes);
+    if (want_lpull && !s->lam2) dalloc_optional(s, &s->lam2, lbytes, true);
     const bool lpull = want_lpull && s->lam2;
     const size_t rn = rec_row(s);
     if (!s->gacc && (rc = dalloc(s, &s->gacc, 3 * rn * tcs))) return rc;

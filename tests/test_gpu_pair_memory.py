@@ -93,3 +93,70 @@ def test_capture_gives_it_back(monkeypatch):
     single.evolve(8)
     assert _bytes(e) == _bytes(single)
     np.testing.assert_array_equal(e.download_post_f(), single.download_post_f())
+
+
+def _single(calls, monkeypatch):
+    monkeypatch.setenv("LB_PAIR", "0")
+    e = _engine(1)
+    for n in calls:
+        e.evolve(n)
+    monkeypatch.setenv("LB_PAIR", "1")
+    return e
+
+
+def test_another_handle_gets_it_back(monkeypatch):
+    """An allocation that the device cannot hold takes what the other handles'
+    pairs hold before it fails; they go on with single steps."""
+    from jyulb import _native
+    single = _single((4, 5), monkeypatch)
+    e = _engine(1)
+    e.evolve(4)
+    assert _bytes(e) > _bytes(single)
+    with pytest.raises(RuntimeError, match="hipMalloc"):  # 320 GB of populations
+        _native.Engine((1290, 1290, 1280), 1, 0.05, (0.0, 0.0, 0.0), (P,) * 6, layout="rows")
+    assert _bytes(e) == _bytes(single) and not e.paired_steps()
+    e.evolve(5)
+    np.testing.assert_array_equal(e.download_post_f(), single.download_post_f())
+
+
+def test_own_allocation_gets_it_back(monkeypatch):
+    """The adjoint's checkpoints on walls at rest."""
+    monkeypatch.setenv("LB_PAIR", "1")
+    e = _engine(0)
+    e.evolve(4)
+    held = _bytes(e)
+    with pytest.raises(RuntimeError, match="hipMalloc"):
+        e.adj_forward(1 << 20, 1, 1, 0)  # terabytes
+    assert _bytes(e) < held and not e.paired_steps()
+    f = e.download_post_f()
+    e.evolve(3)
+    assert not np.array_equal(e.download_post_f(), f)
+
+
+def test_handles_in_other_threads_keep_theirs_while_they_use_it(monkeypatch):
+    """Handles stepping in two threads while a third one's allocations fail."""
+    import threading
+    from jyulb import _native
+    calls = [6] * 40
+    single = _single(calls, monkeypatch)
+    engines = [_engine(1) for _ in range(2)]
+
+    def steps(e):
+        for n in calls:
+            e.evolve(n)
+            e.synchronize()
+
+    def fail():
+        for _ in range(10):
+            try:
+                _native.Engine((1290, 1290, 1280), 1, 0.05, (0.0, 0.0, 0.0), (P,) * 6, layout="rows")
+            except RuntimeError:
+                pass
+
+    threads = [threading.Thread(target=steps, args=(e,)) for e in engines] + [threading.Thread(target=fail)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for e in engines:
+        np.testing.assert_array_equal(e.download_post_f(), single.download_post_f())
