@@ -1734,6 +1734,19 @@ static int layout_arrays(lb_solver* s, int layout) {
     return LB_OK;
 }
 
+// Whether the paired steps' second array leaves a quarter of the device's
+// memory free: what else the program allocates then (torch tensors, another
+// solver's fields) finds room as if it were not there.
+static bool pair_room(const lb_solver* s) {
+    if (s->pair > 0 || s->pull_active) return true;  // asked for, or there anyway
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return avail >= total / 4 + (s->f2 ? 0 : (size_t)s->fsize * ts_size(s->prec));
+}
+
 // The second array of a dense pull-step candidate that was not chosen.
 static void drop_pull_candidate(lb_solver* s) {
     if (s->f2 && !s->pull_active && !s->pair_on && !s->pair_tune) dfree(s, &s->f2, (size_t)s->fsize * ts_size(s->prec));
@@ -2097,6 +2110,7 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
     if (s->sparse && (rc = build_sparse(s))) return rc;
     if (s->sparse) s->pair_on = pair_wanted(s);
     if (s->pair_tune) s->pair_on = true;  // finalized again
+    if (s->pair_on && !pair_room(s)) s->pair_on = s->pair_tune = false;
     if (s->pair_on) pair_tiling(s);
     if (s->pair_on && s->moving && (rc = pair_walls(s))) return rc;
     if (s->pair_on) {
@@ -2269,7 +2283,7 @@ static bool pairs_ready(lb_solver* s) {
     if (pairs_barred(s)) return false;
     if (s->f2) return true;
     const size_t fb = (size_t)s->fsize * ts_size(s->prec);
-    dalloc_optional(s, &s->f2, fb);
+    if (pair_room(s)) dalloc_optional(s, &s->f2, fb);
     if (s->f2 && s->prec == LB_FP16_STORAGE)  // the FP16 guard reads more than the fluid sites
         k_fill<uint64_t><<<(unsigned)((fb / 8 + 255) / 256), 256, 0, s->stream>>>((uint64_t*)s->f2, fb / 8, 0);
     if (!s->f2) drop_pairs(s);

@@ -160,3 +160,31 @@ def test_handles_in_other_threads_keep_theirs_while_they_use_it(monkeypatch):
         t.join()
     for e in engines:
         np.testing.assert_array_equal(e.download_post_f(), single.download_post_f())
+
+
+def test_pairs_leave_a_quarter_of_the_device_free(monkeypatch):
+    """Where less would be left, steps are single, whether the memory goes
+    before or after the set-up; LB_PAIR=1 does not ask."""
+    import torch
+    monkeypatch.delenv("LB_PAIR", raising=False)
+    free = _engine(0)
+    free.evolve(4)
+    assert free.paired_steps()
+    late = _engine(0)
+    total = torch.cuda.mem_get_info()[1]
+    fill = torch.empty(int(0.8 * total), dtype=torch.uint8, device="cuda")
+    try:
+        early = _engine(0)
+        early.evolve(4)
+        late.evolve(4)
+        assert not early.paired_steps() and not late.paired_steps()
+        assert _bytes(early) == _bytes(late) < _bytes(free)
+        monkeypatch.setenv("LB_PAIR", "1")
+        forced = _engine(0)
+        forced.evolve(4)
+        assert forced.paired_steps()
+    finally:
+        del fill
+        torch.cuda.empty_cache()
+    for e in (early, late, forced):
+        np.testing.assert_array_equal(e.download_post_f(), free.download_post_f())
