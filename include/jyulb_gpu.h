@@ -304,6 +304,13 @@ int lb_pull_steps(lb_solver *s, int *on);
  * environment decides instead. Results are identical either way. */
 int lb_paired_steps(lb_solver *s, int *on);
 
+/* Device memory that the handle holds for paired steps only: the second
+ * population array and, with moving walls, 12 bytes per cell. A device
+ * allocation of any handle of the process that would fail takes it back (the
+ * steps stay single until the next lb_finalize), and pairs run only where a
+ * quarter of the device's memory stays free with it (LB_PAIR=1: always). */
+int lb_pair_bytes(lb_solver *s, uint64_t *bytes);
+
 /* The population layout in use (LB_LAYOUT_*; LB_LAYOUT_AUTO until the first
  * lb_finalize resolves it). */
 int lb_layout(lb_solver *s, int *layout);

@@ -3340,6 +3340,13 @@ int lb_paired_steps(lb_solver* s, int* on) {
     return LB_OK;
 }
 
+int lb_pair_bytes(lb_solver* s, uint64_t* bytes) {
+    if (!s || !bytes) return fail(LB_EINVAL, "null argument");
+    std::lock_guard<std::recursive_mutex> lock(s->mx);
+    *bytes = pair_bytes(s);
+    return LB_OK;
+}
+
 int lb_pull_steps(lb_solver* s, int* on) {
     if (!s || !on) return fail(LB_EINVAL, "null argument");
     *on = s->pull_active ? 1 : 0;

@@ -96,6 +96,7 @@ def lib():
         "lb_sparse_codes": ([H, ctypes.POINTER(ctypes.c_uint64)], ctypes.c_int),
         "lb_pull_steps": ([H, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "lb_paired_steps": ([H, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
+        "lb_pair_bytes": ([H, ctypes.POINTER(ctypes.c_uint64)], ctypes.c_int),
         "lb_synchronize": ([H], ctypes.c_int),
         "lb_set_face_data_device": ([H, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p], ctypes.c_int),
         "lb_objective": ([H, ctypes.c_int, ctypes.c_int, dp], ctypes.c_int),
@@ -352,6 +353,13 @@ class Engine:
         v = ctypes.c_int()
         self.call("lb_paired_steps", ctypes.byref(v))
         return bool(v.value)
+
+    def pair_bytes(self):
+        """Device memory that only paired steps use, and that an allocation which
+        needs it gets back."""
+        v = ctypes.c_uint64()
+        self.call("lb_pair_bytes", ctypes.byref(v))
+        return int(v.value)
 
     def layout(self):
         """Name of the population layout in use ("auto" until finalize resolves it)."""

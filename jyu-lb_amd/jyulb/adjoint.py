@@ -47,7 +47,8 @@ def _finish(solver, steps):
 
 def checkpoint_interval(solver, steps, budget_bytes=None, objective="flux"):
     """The checkpoint interval with the least recomputation whose device
-    memory fits in `budget_bytes` (default: half of the free device memory).
+    memory fits in `budget_bytes` (default: half of the free device memory, with
+    what the solver's paired steps hold, which the adjoint's arrays get back).
 
     With n segments of length i = ceil(steps / n) the reverse pass recomputes
     all but the last segment; the fewest segments that fit are the fastest
@@ -83,7 +84,7 @@ def checkpoint_interval(solver, steps, budget_bytes=None, objective="flux"):
         raise ValueError('steps must be >= 1')
     if budget_bytes is None:
         import torch
-        budget_bytes = torch.cuda.mem_get_info()[0] // 2
+        budget_bytes = (torch.cuda.mem_get_info()[0] + eng.pair_bytes()) // 2
 
     def need(i):
         return (-(-steps // i) + 1) * fb + min(i, steps) * rb + extra

@@ -188,3 +188,22 @@ def test_pairs_leave_a_quarter_of_the_device_free(monkeypatch):
         torch.cuda.empty_cache()
     for e in (early, late, forced):
         np.testing.assert_array_equal(e.download_post_f(), free.download_post_f())
+
+
+def test_checkpoint_interval_does_not_depend_on_pairs(monkeypatch):
+    """interval='auto' budgets the free memory: here of a device that holds 60
+    population arrays, of which the pairs' is one."""
+    import torch
+    from types import SimpleNamespace
+    from jyulb import adjoint
+    monkeypatch.setenv("LB_PAIR", "1")
+    e = _engine(0)
+    single = _bytes(e)
+    array = 19 * 8 * LAT[0] * LAT[1] * 64
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda: (60 * array - (_bytes(e) - single), 1 << 38))
+    solver = SimpleNamespace(engine=e)
+    before = [adjoint.checkpoint_interval(solver, n) for n in range(50, 600, 50)]
+    assert e.pair_bytes() == 0
+    e.evolve(6)
+    assert e.pair_bytes() == _bytes(e) - single > 0
+    assert [adjoint.checkpoint_interval(solver, n) for n in range(50, 600, 50)] == before
