@@ -1616,6 +1616,24 @@ static bool pair_wanted(const lb_solver* s) {
     return 3 * (uint64_t)s->d.ny * (uint64_t)s->rs * ts + Q * (uint64_t)s->ps * ts < (1ull << 32);
 }
 
+// Without timing (LB_AUTOTUNE=0): whether a lattice steps in pairs that
+// tune_pair would settle. The lines lie where pairs were never slower (ms per
+// step, single / paired). Moving lid: FP64 from 24^3 0.0078 / 0.0057 over 64^3
+// 0.0162 / 0.0160 to 256^3 0.954 / 0.628; FP32 64^3 0.0108 / 0.0123, 70^3
+// 0.0210 / 0.0139, 512x128x128 0.266 / 0.195; FP32 storage 64x64x256 0.0349 /
+// 0.0427, 100x100x100 0.0457 / 0.0407, 512x128x128 0.305 / 0.234; FP16 64^3
+// 0.0115 / 0.0134, 256^3 0.295 / 0.359. Sparse with a lid over 20% solid:
+// FP64 384x192x192 0.615 / 0.522, FP32 320^3 0.867 / 0.688. Walls at rest in
+// FP16: 64^3 0.0193 / 0.0123, 256^3 0.280 / 0.272, 320^3 0.532 / 0.532.
+static bool pair_untimed(const lb_solver* s) {
+    switch (s->prec) {
+    case LB_FP64: return true;
+    case LB_FP32_SHIFTED: return s->ncell > (1 << 18);
+    case LB_FP32_STORAGE: return s->ncell > (1 << 20);
+    default: return !s->moving && s->ncell <= (1 << 24);
+    }
+}
+
 // The tiling of the paired steps: inner columns along k and j, planes per
 // workgroup. A workgroup runs two iterations more than it stores planes, and
 // about one more to start; a CU holds one workgroup at a time, so a launch
@@ -2121,11 +2139,12 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
         // cavities 256^3 FP64 0.928 / 0.624, FP32 0.501 / 0.343, FP16 0.284 /
         // 0.389, 64^3 FP64 0.0164 / 0.0171, 48^3 FP64 0.0128 / 0.0102; 64^3
         // channel FP16 0.0184 / 0.0112. Sparse FP32: see pair_wanted.
-        s->pair_tune = s->pair < 0 && s->autotune &&
-                       (s->moving || s->prec == LB_FP16_STORAGE ||
-                        (s->sparse && s->prec != LB_FP64 && s->nfluid < (1 << 23)));
+        const bool depends = s->pair < 0 && (s->moving || s->prec == LB_FP16_STORAGE ||
+                                             (s->sparse && s->prec != LB_FP64 && s->nfluid < (1 << 23)));
+        s->pair_tune = depends && s->autotune;
+        if (depends && !s->autotune && !pair_untimed(s)) drop_pairs(s);
         if (s->pair_tune) s->pair_on = false;
-        else s->tune = false;  // few single steps are left to tune
+        else if (s->pair_on) s->tune = false;  // few single steps are left to tune
     }
     if (s->prec == LB_FP16_STORAGE && s->f16_auto) {
         k_maxdev<<<256, 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->nq, s->rho0, s->part);

@@ -134,3 +134,30 @@ def test_single_steps_launches_on_lattices_that_pair(name, env, monkeypatch):
         if k.startswith("f_"):
             a, b = a[:, fluid[0], fluid[1], fluid[2]], b[:, fluid[0], fluid[1], fluid[2]]
         np.testing.assert_array_equal(b, a, err_msg=f"{name} {k}")
+
+
+@pytest.mark.parametrize("lat,precision,lid,pairs", [
+    ((24, 20, 40), "fp64", True, True),
+    ((64, 64, 64), "fp32", True, False), ((66, 64, 64), "fp32", True, True),
+    ((64, 64, 256), "fp32_storage", True, False), ((65, 64, 256), "fp32_storage", True, True),
+    ((24, 20, 40), "fp16", True, False), ((24, 20, 40), "fp16", False, True),
+    ((24, 20, 40), "fp32", False, True), ((24, 20, 40), "fp32_storage", False, True),
+])
+def test_untimed_choice(lat, precision, lid, pairs, monkeypatch):
+    """LB_AUTOTUNE=0 times nothing: pairs where they are never slower, single
+    steps elsewhere, from the first call on."""
+    from jyulb import _native
+    monkeypatch.delenv("LB_PAIR", raising=False)
+    monkeypatch.setenv("LB_AUTOTUNE", "0")
+    e = _native.Engine(lat, 1, 0.05, (1e-6, 0.0, 0.0), (P, P, W, W, W, W), precision=precision, layout="rows")
+    phase, vel = np.ones(lat, dtype=np.uint8), np.zeros(lat + (3,))
+    if lid:
+        phase[:, :, -1] = 0
+        vel[:, :, -1, 0] = 0.05
+    e.upload_phase(phase)
+    e.upload_den_vel(np.ones(lat), vel)
+    e.finalize()
+    held = e.info()["device_bytes"]
+    e.evolve(30)
+    assert e.paired_steps() == pairs
+    assert (e.info()["device_bytes"] > held) == pairs
