@@ -31,6 +31,7 @@
 #include <stdarg.h>
 #include <algorithm>
 #include <atomic>
+#include <functional>
 #include <utility>
 #include <vector>
 #include <stdio.h>
@@ -2144,7 +2145,6 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
         s->pair_tune = depends && s->autotune;
         if (depends && !s->autotune && !pair_untimed(s)) drop_pairs(s);
         if (s->pair_tune) s->pair_on = false;
-        else if (s->pair_on) s->tune = false;  // few single steps are left to tune
     }
     if (s->prec == LB_FP16_STORAGE && s->f16_auto) {
         k_maxdev<<<256, 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->nq, s->rho0, s->part);
@@ -2309,6 +2309,9 @@ static bool pairs_ready(lb_solver* s) {
     return s->pair_on;
 }
 
+// Whether evolve calls step in pairs.
+static bool pairs_used(const lb_solver* s) { return s->pair_on && !s->captured && !(s->moving && !s->mov_pairs); }
+
 static void swap_rho(PairParams& q) {
     const double* in = q.rho_out;
     q.rho_out = const_cast<double*>(q.rho_in);
@@ -2424,8 +2427,11 @@ static int tune_candidates(const lb_solver* s, StepCfg* c) {
 // 512x128x128 duct FP64 0.465 / 0.452, FP16 0.152 / 0.159; the dense
 // 768x384x384 medium FP64 7.06 / 7.48, FP16 2.22 / 2.48.
 constexpr int TUNE_PULL_STEPS = 2 * TUNE_STEPS + 1;
-static int tune_pull(lb_solver* s) {
-    if (!s->f2 || s->pull_active) return LB_OK;
+// How the tuner steps: run(n) takes n of the caller's steps, all single;
+// ready(n) goes where the next n can be timed together.
+using StepsFn = std::function<int(uint32_t)>;
+static int tune_pull(lb_solver* s, const StepsFn& ready, const StepsFn& run) {
+    if (!s->f2 || s->pull_active || s->sparse) return LB_OK;
     if (s->captured) {  // pull steps leave the state in the other array too (pairs_barred)
         drop_pull_candidate(s);
         return LB_OK;
@@ -2435,17 +2441,17 @@ static int tune_pull(lb_solver* s) {
     for (hipEvent_t& e : ev) ok = ok && hipEventCreate(&e) == hipSuccess;
     int rc = LB_OK;
     float ms_aa = 0.0f, ms_pull = 0.0f;
-    if (ok) {
+    if (ok && !(rc = ready(TUNE_STEPS))) {
         HIPCHK(hipEventRecord(ev[0], s->stream));
-        rc = run_steps(s, TUNE_STEPS, false);
+        rc = run(TUNE_STEPS);
         if (!rc) {
             HIPCHK(hipEventRecord(ev[1], s->stream));
             s->pull_active = true;
-            rc = run_steps(s, 1, false);  // reaches the state pull steps start from
+            rc = run(1);  // reaches the state pull steps start from
         }
-        if (!rc) {
+        if (!rc && !(rc = ready(TUNE_STEPS))) {
             HIPCHK(hipEventRecord(ev[2], s->stream));
-            rc = run_steps(s, TUNE_STEPS, false);
+            rc = run(TUNE_STEPS);
         }
         if (!rc) {
             HIPCHK(hipEventRecord(ev[3], s->stream));
@@ -2460,15 +2466,15 @@ static int tune_pull(lb_solver* s) {
     for (hipEvent_t e : ev)
         if (e) (void)hipEventDestroy(e);
     s->pull_active = ok && !rc && ms_pull < (1.0f - TUNE_MARGIN) * ms_aa;
-    if (!s->sparse) drop_pull_candidate(s);  // the state is in s->f either way
+    drop_pull_candidate(s);  // the state is in s->f either way
     return rc;
 }
 
-static int tune_step(lb_solver* s) {
+static int tune_step(lb_solver* s, const StepsFn& ready, const StepsFn& run) {
     StepCfg c[TUNE_MAX];
     const int n = tune_candidates(s, c);
     s->tune = false;
-    if (n < 2) return tune_pull(s);
+    if (n < 2) return tune_pull(s, ready, run);
     std::vector<hipEvent_t> ev(2 * n, nullptr);
     for (hipEvent_t& e : ev)
         if (hipEventCreate(&e) != hipSuccess) e = nullptr;
@@ -2476,17 +2482,19 @@ static int tune_step(lb_solver* s) {
         if (!e) {
             for (hipEvent_t x : ev)
                 if (x) (void)hipEventDestroy(x);
-            return tune_pull(s);  // no timing: keep the default (and the in-place steps)
+            return tune_pull(s, ready, run);  // no timing: keep the default (and the in-place steps)
         }
-    int rc = run_steps(s, TUNE_WARM, false);
+    int rc = ready(TUNE_WARM);
+    if (!rc) rc = run(TUNE_WARM);
     for (int i = 0; i < n && !rc; ++i) {
         s->step_tile = c[i].tile;
         s->step_lds[0] = c[i].lds_even;
         s->step_lds[1] = c[i].lds_odd;
         s->xcd_cells = c[i].xcd_cells;
         s->xcd_chunk = c[i].chunk;
+        if ((rc = ready(TUNE_STEPS))) break;
         HIPCHK(hipEventRecord(ev[2 * i], s->stream));
-        rc = run_steps(s, TUNE_STEPS, false);
+        rc = run(TUNE_STEPS);
         HIPCHK(hipEventRecord(ev[2 * i + 1], s->stream));
     }
     if (rc) {
@@ -2521,7 +2529,26 @@ static int tune_step(lb_solver* s) {
     s->step_lds[1] = c[best].lds_odd;
     s->xcd_cells = c[best].xcd_cells;
     s->xcd_chunk = c[best].chunk;
-    return tune_pull(s);
+    return tune_pull(s, ready, run);
+}
+
+// Steps that tune_step takes of a pass with a checkpoint every `interval`
+// steps, which its timed steps do not cross.
+static uint64_t tune_extent(const lb_solver* s, uint32_t interval) {
+    if (interval < TUNE_STEPS) return UINT64_MAX;
+    StepCfg c[TUNE_MAX];
+    const int n = tune_candidates(s, c);
+    uint64_t at = 0;
+    auto block = [&](uint32_t len) {
+        const uint32_t left = interval - (uint32_t)(at % interval);
+        at += (left < len ? left : 0) + len;
+    };
+    block(TUNE_WARM);
+    for (int i = 0; i < n; ++i) block(TUNE_STEPS);
+    block(TUNE_STEPS);
+    block(1);
+    block(TUNE_STEPS);
+    return at;
 }
 
 // Single or paired steps, by timing the call's own: PAIR_TUNE single steps and
@@ -2584,7 +2611,7 @@ static int evolve_steps(lb_solver* s, uint32_t steps) {
     const bool barred = pairs_barred(s);
     if (s->prec == LB_FP16_STORAGE && (s->f16_dirty || s->f16_since >= s->f16_check) && (rc = fp16_guard(s)))
         return rc;
-    if (s->tune) {
+    if (s->tune && !pairs_used(s)) {
         // tuning takes TUNE_WARM + TUNE_STEPS per candidate of this call's
         // steps; a shorter call leaves it to a later one
         StepCfg c[TUNE_MAX];
@@ -2594,7 +2621,8 @@ static int evolve_steps(lb_solver* s, uint32_t steps) {
             s->tune = false;
         } else if (steps > (uint32_t)(TUNE_WARM + n * TUNE_STEPS + np)) {
             const uint64_t before = s->steps;
-            if ((rc = tune_step(s))) return rc;
+            if ((rc = tune_step(s, [](uint32_t) { return LB_OK; }, [&](uint32_t k) { return run_steps(s, k, false); })))
+                return rc;
             steps -= (uint32_t)(s->steps - before);
         }
     }
@@ -3107,15 +3135,21 @@ int lb_adj_forward(lb_solver* s, uint32_t steps, uint32_t interval, int face, in
     }
     s->adj_po = s->next_odd;
     s->ckpt_odd.assign(nseg + 1, 1);
-    StepParams p = params(s);
-    for (uint32_t seg = 0; seg < nseg; ++seg) {
-        HIPCHK(stream_copy((char*)s->ckpt + (size_t)seg * fbytes, s->f, fbytes, s->stream));
-        s->ckpt_odd[seg] = (uint8_t)s->next_odd;
-        const uint32_t len = std::min(interval, steps - seg * interval);
-        for (uint32_t t = 0; t < len; ++t) {
-            p.store_dv = (seg * interval + t + 1 == steps) ? 1 : 0;
+    StepParams p;
+    uint32_t g = 0, stored = 0;  // steps taken, checkpoints stored
+    auto checkpoint = [&]() -> int {  // where a segment starts
+        if (g % interval || stored > g / interval) return LB_OK;
+        HIPCHK(stream_copy((char*)s->ckpt + (size_t)stored * fbytes, s->f, fbytes, s->stream));
+        s->ckpt_odd[stored++] = (uint8_t)s->next_odd;
+        return LB_OK;
+    };
+    auto advance = [&](uint32_t n) -> int {
+        p = params(s);
+        for (; n; --n, ++g) {
+            if (int e = checkpoint()) return e;
+            p.store_dv = g + 1 == steps ? 1 : 0;
             // the last segment records (rho, u*) as the reverse pass's recompute would
-            p.rec = seg + 1 == nseg ? (char*)s->rec + (size_t)t * 4 * rec_row(s) * tcs : nullptr;
+            p.rec = g / interval + 1 == nseg ? (char*)s->rec + (size_t)(g % interval) * 4 * rec_row(s) * tcs : nullptr;
             if (diss && p.store_dv) {  // the objective is on the final step's collision input
                 StepParams q = p;
                 q.rec = nullptr;
@@ -3127,7 +3161,21 @@ int lb_adj_forward(lb_solver* s, uint32_t steps, uint32_t interval, int face, in
             one_step(s, p, s->next_odd);
             s->steps++;
         }
+        return LB_OK;
+    };
+    // The launch of single steps is tuned here where evolve calls, which step
+    // in pairs, leave it untuned (512x128x128 duct in FP64: 0.504 ms per step
+    // untuned, 0.486 tuned). No timed step crosses a checkpoint.
+    if (s->tune && pairs_used(s) && steps > tune_extent(s, interval)) {
+        auto ready = [&](uint32_t n) -> int {
+            const uint32_t left = interval - g % interval;
+            if (left < n)
+                if (int e = advance(left)) return e;
+            return checkpoint();
+        };
+        if ((rc = tune_step(s, ready, advance))) return rc;
     }
+    if ((rc = advance(steps - g))) return rc;
     HIPCHK(hipGetLastError());
     HIPCHK(stream_copy((char*)s->ckpt + (size_t)nseg * fbytes, s->f, fbytes, s->stream));
     s->ckpt_odd[nseg] = (uint8_t)s->next_odd;
@@ -3355,7 +3403,7 @@ int lb_sparse_codes(lb_solver* s, uint64_t* counts) {
 
 int lb_paired_steps(lb_solver* s, int* on) {
     if (!s || !on) return fail(LB_EINVAL, "null argument");
-    *on = s->pair_on && !s->captured && !(s->moving && !s->mov_pairs) ? 1 : 0;
+    *on = pairs_used(s) ? 1 : 0;
     return LB_OK;
 }
 

@@ -555,3 +555,35 @@ def test_dissipation_objective_torch_function():
     assert abs(float(J.detach()) - J0) <= 1e-14 * abs(J0)
     np.testing.assert_allclose(a.grad.cpu().numpy(), ga0, rtol=0, atol=1e-14 * np.max(np.abs(ga0)))
     np.testing.assert_allclose(v.grad.cpu().numpy(), gf0, rtol=0, atol=1e-14 * np.max(np.abs(gf0)))
+
+
+@pytest.mark.parametrize("interval", [120, 60, 7, 3])
+@pytest.mark.parametrize("layout", ["rows", "sparse"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_adjoint_tunes_the_launch_that_evolve_in_pairs_does_not_use(precision, layout, interval, monkeypatch, capfd):
+    """Where evolve steps in pairs, the adjoint's single steps choose their own
+    launch, on the forward pass's steps: the same objective and gradients, with
+    every length of the segments; not where a segment is shorter than what one
+    candidate takes."""
+    monkeypatch.setenv("LB_PAIR", "1")
+    monkeypatch.setenv("LB_AUTOTUNE_MIN_CELLS", "0")
+    monkeypatch.setenv("LB_AUTOTUNE_VERBOSE", "1")
+    out = []
+    for tune in ("0", "1"):
+        monkeypatch.setenv("LB_AUTOTUNE", tune)
+        s, prof, amp = make_channel(TRT, precision, seed=8, layout=layout)
+        acc, fden, fvel, g = _inputs(s)
+        s.engine.evolve(60)
+        assert s.engine.paired_steps()
+        capfd.readouterr()
+        s.engine.snapshot()
+        out.append(_adjoint(s, acc, fden, fvel, g, 120, interval))
+        log = capfd.readouterr().err
+        print(log)
+        assert ("step launch" in log) == (tune == "1" and interval > 3)
+        s.engine.restore()
+        s.engine.evolve(9)
+        out[-1] = out[-1] + (s.engine.download_post_f(),)
+    assert out[0][0] == out[1][0]
+    for a, b in zip(out[0][1:], out[1][1:]):
+        np.testing.assert_array_equal(a, b)
