@@ -1443,7 +1443,6 @@ static int count_mask(lb_solver* s, int64_t* nfluid, int64_t* nmoving) {
                                                                   s->ladd_u, s->mov_cell, cnt);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s->stream));
-        if (s->finalized && (s->pair_on || s->pair_tune) && (rc = pair_walls(s))) return rc;  // else at lb_finalize's end
     }
     return LB_OK;
 }
@@ -1799,6 +1798,40 @@ static bool give_back(lb_solver* s) {
     return true;
 }
 
+// Single or paired steps for the lattice and the walls as they are, or to be
+// settled by timing (tune_pair), with single steps until then. Pairs are faster
+// where walls stand still and values have 4 bytes or more (ms per step, single
+// / paired: 256^3 channel FP64 0.894 / 0.567, FP32 0.451 / 0.300; 48^3 FP64
+// 0.0215 / 0.0085). With moving walls or FP16 storage, where the collisions
+// bind, it depends (figures at pair_untimed). Sparse FP32: see pair_wanted.
+static int settle_pairs(lb_solver* s) {
+    s->pair_tune = false;
+    s->pair_on = pair_wanted(s) && pair_room(s);
+    if (s->pair_on) pair_tiling(s);
+    if (s->pair_on && s->pair < 0 &&
+        (s->moving || s->prec == LB_FP16_STORAGE ||
+         (s->sparse && s->prec != LB_FP64 && s->nfluid < (1 << 23)))) {
+        s->pair_tune = s->autotune;
+        s->pair_on = !s->autotune && pair_untimed(s);
+    }
+    if (!s->pair_on && !s->pair_tune) {
+        drop_pairs(s);
+        return LB_OK;
+    }
+    return s->moving ? pair_walls(s) : LB_OK;
+}
+
+// Wall velocities changed: whether walls move, the palette, and, where walls
+// start or stop moving, the choice of the steps, unless pairs are in use and
+// are never slower.
+static int walls_changed(lb_solver* s, bool moving) {
+    const bool other = moving != s->moving;
+    s->moving = moving;
+    if (!s->finalized) return LB_OK;  // lb_finalize settles it
+    if (other && !(s->pair_on && (s->pair > 0 || pair_untimed(s)))) return settle_pairs(s);
+    return moving && (s->pair_on || s->pair_tune) ? pair_walls(s) : LB_OK;
+}
+
 int lb_create(const lb_config* cfg, lb_solver** out) {
     if (!cfg || !out) return fail(LB_EINVAL, "null argument");
     *out = nullptr;
@@ -2127,25 +2160,7 @@ int lb_finalize(lb_solver* s, int64_t* nfluid) {
         if ((rc = layout_arrays(s, layout))) return rc;
     }
     if (s->sparse && (rc = build_sparse(s))) return rc;
-    if (s->sparse) s->pair_on = pair_wanted(s);
-    if (s->pair_tune) s->pair_on = true;  // finalized again
-    if (s->pair_on && !pair_room(s)) s->pair_on = s->pair_tune = false;
-    if (s->pair_on) pair_tiling(s);
-    if (s->pair_on && s->moving && (rc = pair_walls(s))) return rc;
-    if (s->pair_on) {
-        // Pairs are faster where walls stand still and values have 4 bytes or
-        // more (ms per step, single / paired: 256^3 channel FP64 0.894 /
-        // 0.567, FP32 0.451 / 0.300; 48^3 FP64 0.0215 / 0.0085). With moving
-        // walls or FP16 storage, where the collisions bind, it depends:
-        // cavities 256^3 FP64 0.928 / 0.624, FP32 0.501 / 0.343, FP16 0.284 /
-        // 0.389, 64^3 FP64 0.0164 / 0.0171, 48^3 FP64 0.0128 / 0.0102; 64^3
-        // channel FP16 0.0184 / 0.0112. Sparse FP32: see pair_wanted.
-        const bool depends = s->pair < 0 && (s->moving || s->prec == LB_FP16_STORAGE ||
-                                             (s->sparse && s->prec != LB_FP64 && s->nfluid < (1 << 23)));
-        s->pair_tune = depends && s->autotune;
-        if (depends && !s->autotune && !pair_untimed(s)) drop_pairs(s);
-        if (s->pair_tune) s->pair_on = false;
-    }
+    if ((rc = settle_pairs(s))) return rc;
     if (s->prec == LB_FP16_STORAGE && s->f16_auto) {
         k_maxdev<<<256, 256, 0, s->stream>>>(s->mask, s->den, s->vel, s->nq, s->rho0, s->part);
         HIPCHK(hipGetLastError());
@@ -2189,8 +2204,7 @@ int lb_refresh_walls(lb_solver* s) {
     if (rc) return rc;
     int64_t nf, nm;
     if ((rc = count_mask(s, &nf, &nm))) return rc;
-    s->moving = nm > 0;
-    return LB_OK;
+    return walls_changed(s, nm > 0);
 }
 
 // Zou-He data bound of |f - w rho0| over the FIXED faces (k_face_bound), 0
@@ -2753,8 +2767,7 @@ static int host_inputs(lb_solver* s, unsigned int hf) {
         int rc = build_mask(s, true);
         if (rc) return rc;
         int64_t nf, nm;
-        if ((rc = count_mask(s, &nf, &nm))) return rc;
-        s->moving = nm > 0;
+        if ((rc = count_mask(s, &nf, &nm)) || (rc = walls_changed(s, nm > 0))) return rc;
     }
     s->acc_on = (hf & SYNC_ACC) != 0;
     return LB_OK;
