@@ -1608,6 +1608,7 @@ static void layout_defaults(lb_solver* s, int layout) {
 static bool pair_wanted(const lb_solver* s) {
     if (s->sp_pull >= 0 || s->pair == 0 || s->captured) return false;
     if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
+    if (s->prec == LB_FP16_STORAGE && s->f16_check < 2) return false;  // every step is checked
     if (s->sparse) {
         const bool prec = s->prec == LB_FP64 || (s->prec == LB_FP32_SHIFTED && (s->autotune || s->nfluid >= (1 << 23)));
         return s->pair > 0 || (prec && s->nfluid >= (1 << 19) && s->nfluid * 10 >= s->ncell * 7);
@@ -2588,7 +2589,7 @@ static int tune_pair(lb_solver* s) {
     for (hipEvent_t e : ev)
         if (e) (void)hipEventDestroy(e);
     s->pair_tune = false;
-    s->pair_on = ok && ms[1] < ms[0];
+    s->pair_on = ok && s->pair_on && ms[1] < ms[0];  // off by now where the second array found no room
     if (s->tune_verbose)
         fprintf(stderr, "[jyulb] single steps %.4f ms, paired steps %.4f ms per step\n", ms[0] / PAIR_TUNE,
                 ms[1] / PAIR_TUNE);
@@ -2640,10 +2641,15 @@ static int evolve_steps(lb_solver* s, uint32_t steps) {
             steps -= (uint32_t)(s->steps - before);
         }
     }
-    if (s->pair_tune && !s->tune && steps > (uint32_t)PAIR_TUNE_STEPS && !barred) {
-        const uint64_t before = s->steps;
-        if ((rc = tune_pair(s))) return rc;
-        steps -= (uint32_t)(s->steps - before);
+    if (s->pair_tune && !s->tune && !barred && !(s->moving && !s->mov_pairs)) {
+        // from the next FP16 check on, where that would fall into the timing
+        const uint32_t wait = s->prec == LB_FP16_STORAGE && s->f16_since + PAIR_TUNE_STEPS > s->f16_check
+                                  ? s->f16_check - std::min(s->f16_since, s->f16_check) : 0u;
+        if (steps > wait + (uint32_t)PAIR_TUNE_STEPS) {
+            const uint64_t before = s->steps;
+            if ((wait && (rc = run_steps(s, wait, false))) || (rc = tune_pair(s))) return rc;
+            steps -= (uint32_t)(s->steps - before);
+        }
     }
     if (s->keep_prev) {
         if ((rc = run_steps(s, steps - 1, false)) || (rc = capture_prev(s)) || (rc = run_steps(s, 1, true)))

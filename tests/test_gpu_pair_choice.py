@@ -43,6 +43,19 @@ class Flow:
 STILL, SAME, OTHER = (0.0, 0.0, 0.0), (0.02, 0.01, 0.0), (0.0, 0.02, 0.0)
 
 
+def test_walls_that_do_not_qualify_wait_for_the_timing(monkeypatch, capfd):
+    """Two velocities at one site: there is nothing to compare. Once they
+    agree, the next long call times both."""
+    s = Flow(monkeypatch).walls(SAME, OTHER)
+    s.e.finalize()
+    assert TIMED not in s.log(capfd, 60)
+    assert not s.e.paired_steps() and s.e.pair_bytes() == 0
+    s.walls(SAME, SAME).e.refresh_walls()
+    assert TIMED not in s.log(capfd, 20)  # too short
+    assert TIMED in s.log(capfd, 60)
+    assert s.e.paired_steps() == (s.e.pair_bytes() > 0)
+
+
 @pytest.mark.parametrize("precision,kept", [("fp64", True), ("fp32", False)])
 def test_walls_that_start_to_move_settle_it_again(precision, kept, monkeypatch, capfd):
     """Pairs go on where they are never slower (FP64); else both are timed."""
@@ -65,3 +78,41 @@ def test_finalized_again_settles_it_again(monkeypatch, capfd):
         assert not s.e.paired_steps()
         assert TIMED in s.log(capfd, 60)
         assert TIMED not in s.log(capfd, 60)
+
+
+def test_no_pairs_where_every_step_is_checked(monkeypatch):
+    s = Flow(monkeypatch, "fp16", LB_PAIR="1", LB_FP16_CHECK="1").walls(STILL, STILL)
+    s.e.finalize()
+    s.e.evolve(6)
+    assert not s.e.paired_steps() and s.e.pair_bytes() == 0
+
+
+def test_no_pairs_where_their_array_finds_no_room_in_the_timing(monkeypatch, capfd):
+    import torch
+    s = Flow(monkeypatch, "fp16").walls(STILL, STILL)
+    s.e.finalize()
+    fill = torch.empty(int(0.8 * torch.cuda.mem_get_info()[1]), dtype=torch.uint8, device="cuda")
+    try:
+        assert TIMED in s.log(capfd, 60)
+    finally:
+        del fill
+        torch.cuda.empty_cache()
+    assert not s.e.paired_steps() and s.e.pair_bytes() == 0
+
+
+@pytest.mark.parametrize("since", [0, 30, 50, 63])
+@pytest.mark.parametrize("velocity", [STILL, SAME], ids=["still", "moving"])
+def test_fp16_checks_stay_where_they_were(since, velocity, monkeypatch, capfd):
+    """The timing waits for the next check of the FP16 values, and changes no
+    bit: the same steps with LB_PAIR=0."""
+    out = []
+    for env in ({"LB_PAIR": "0"}, {}):
+        s = Flow(monkeypatch, "fp16", **env).walls(velocity, velocity)
+        s.e.finalize()
+        for _ in range(since):
+            s.e.evolve(1)
+        log = s.log(capfd, 60) + s.log(capfd, 70)
+        assert (TIMED in log) == (not env)
+        out.append((s.e.download_post_f(), *s.e.download_den_vel(), s.e.info()["fp16_scale"]))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
