@@ -27,6 +27,7 @@
 // lb_kernels.h (lb_inst.hip).
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
+#include <limits.h>
 #include <math.h>
 #include <stdarg.h>
 #include <algorithm>
@@ -1605,16 +1606,48 @@ static void layout_defaults(lb_solver* s, int layout) {
 // from 2^23 sites (768x384x384 2.57 / 2.28), which below lets tune_pair time
 // both; FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 /
 // 0.561) stay single.
+static bool pair_thin(const lb_solver* s);
 static bool pair_wanted(const lb_solver* s) {
     if (s->sp_pull >= 0 || s->pair == 0 || s->captured) return false;
     if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
     if (s->prec == LB_FP16_STORAGE && s->f16_check < 2) return false;  // every step is checked
+    if (s->pair < 0 && pair_thin(s)) return false;
     if (s->sparse) {
         const bool prec = s->prec == LB_FP64 || (s->prec == LB_FP32_SHIFTED && (s->autotune || s->nfluid >= (1 << 23)));
         return s->pair > 0 || (prec && s->nfluid >= (1 << 19) && s->nfluid * 10 >= s->ncell * 7);
     }
     const uint64_t ts = ts_size(s->prec);
     return 3 * (uint64_t)s->d.ny * (uint64_t)s->rs * ts + Q * (uint64_t)s->ps * ts < (1ull << 32);
+}
+
+// Lattices too thin for the sweep along i to pay. However few columns a plane
+// has, an iteration takes over 2 us, so that 256 CUs take 4.4 to 5 ns per plane
+// and step, where a wave of 64 cells in a single step takes 1.1 to 1.7 ns; short
+// lattices wait for the launch either way. Dense: the most planes that pairs
+// take, by waves per plane, between these times (ms per step, single / paired).
+// One wave: FP64 1024x1x64 0.012 / 0.008, 4096x1x64 0.021 / 0.022; FP32 0.010 /
+// 0.008, 0.014 / 0.022. Two (2x4): FP64 4096 0.029 / 0.022, 16384 0.068 / 0.074;
+// FP32 1024 0.015 / 0.008, 4096 0.021 / 0.022. Three (3x20): FP64 65536 0.414 /
+// 0.284, FP32 0.303 / 0.298; FP16 4096 0.027 / 0.024, 16384 0.067 / 0.084. Four:
+// FP16 16384 0.0845 / 0.0842, 65536 0.319 / 0.327.
+// In the sparse layout, whose single steps see compact sites only, also where
+// an axis is a few cells and the rims are as much again (20% solid, periodic:
+// FP64 2000x2000x1 0.186 / 0.273, 3x1000x1000 0.133 / 0.149, 4x512x512 0.050 /
+// 0.048; FP32 4x2500x2500 0.605 / 0.647, 5x1300x2500 0.446 / 0.396) or a plane
+// has fewer cells than half a tile (FP64 16384x12x12 0.098 / 0.108, 16384x16x16
+// 0.181 / 0.156; FP32 65536x16x16 0.416 / 0.472, 65536x20x20 0.690 / 0.536).
+static bool pair_thin(const lb_solver* s) {
+    const Dims& d = s->d;
+    if (s->sparse) {
+        const bool fp64 = s->prec == LB_FP64;
+        return std::min({d.nx, d.ny, d.nz}) < (fp64 ? 4 : 5) || (int64_t)d.ny * d.nz < (fp64 ? 256 : 400);
+    }
+    constexpr int MOST[4][4] = {{2400, 10000, INT_MAX, INT_MAX},  // LB_FP64
+                                {1700, 3700, INT_MAX, INT_MAX},   // LB_FP32_SHIFTED
+                                {1400, 3500, 6000, 16384},        // LB_FP16_STORAGE
+                                {1600, 6400, INT_MAX, INT_MAX}};  // LB_FP32_STORAGE
+    const int64_t waves = (int64_t)d.ny * (d.nzp / 64);
+    return waves <= 4 && d.nx > MOST[s->prec][waves - 1];
 }
 
 // Without timing (LB_AUTOTUNE=0): whether a lattice steps in pairs that

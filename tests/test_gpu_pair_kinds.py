@@ -161,3 +161,35 @@ def test_untimed_choice(lat, precision, lid, pairs, monkeypatch):
     e.evolve(30)
     assert e.paired_steps() == pairs
     assert (e.info()["device_bytes"] > held) == pairs
+
+
+@pytest.mark.parametrize("lat,precision,layout,pairs", [
+    ((1024, 1, 1), "fp64", "rows", True), ((4096, 1, 1), "fp64", "rows", False), ((4096, 2, 4), "fp64", "rows", True),
+    ((8192, 2, 4), "fp32_storage", "rows", False), ((8192, 3, 4), "fp32_storage", "rows", True),
+    ((4096, 1, 64), "fp32", "soa", False), ((4096, 1, 200), "fp32", "soa", True), ((1, 4096, 1), "fp32", "rows", True),
+    ((900, 800, 1), "fp64", "sparse", False), ((1, 800, 900), "fp64", "sparse", False),
+    ((420, 4, 420), "fp64", "sparse", True), ((4000, 12, 14), "fp64", "sparse", False),
+    ((2800, 16, 16), "fp64", "sparse", True),
+])
+def test_thin_lattices(lat, precision, layout, pairs, monkeypatch):
+    """Lattices of which the planes are too thin for the pairs' sweep step
+    singly, and the same bits either way."""
+    from jyulb import _native
+    rng = np.random.default_rng(2)
+    phase = (rng.random(lat) > (0.15 if layout == "sparse" else 0.01)).astype(np.uint8)
+    out = []
+    for pair in (None, "1", "0"):
+        monkeypatch.delenv("LB_PAIR", raising=False)
+        if pair:
+            monkeypatch.setenv("LB_PAIR", pair)
+        print(f"{lat} {precision} {layout} LB_PAIR={pair}", flush=True)
+        e = _native.Engine(lat, 1, 0.05, (1e-6, 2e-6, 0.0), (P,) * 6, precision=precision, layout=layout)
+        e.upload_phase(phase)
+        e.upload_den_vel(1.0 + 0.01 * np.random.default_rng(3).standard_normal(lat), np.zeros(lat + (3,)))
+        e.finalize()
+        e.evolve(7)
+        assert e.paired_steps() == (pairs if pair is None else pair == "1")
+        out.append((e.download_post_f(), *e.download_den_vel()))
+    for a, b, c in zip(*out):
+        np.testing.assert_array_equal(a, c)
+        np.testing.assert_array_equal(b, c)
