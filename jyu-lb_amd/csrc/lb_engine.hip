@@ -819,7 +819,7 @@ struct lb_solver {
     uint8_t* st_phase = nullptr;
     double *st_den = nullptr, *st_vel = nullptr, *st_acc = nullptr;
     int64_t ncnt = 0;
-    bool h_pinned = false;             // kernels read and write the host fields themselves (k_host_in)
+    bool h_pinned = false;             // kernels read and write the host fields themselves (pinned_rows)
     unsigned int* in_flags = nullptr;  // SYNC_* of k_host_in, zero between calls, and their place on the host
     unsigned int* h_flags = nullptr;
     // FP16 storage guard: steps between checks of the stored magnitudes, steps
@@ -2734,6 +2734,17 @@ static bool pinned(const void* p, size_t n) {
     return true;
 }
 
+// Whether kernels reach the host fields in place as fast as staged copies do:
+// each row is requests of its own over the bus, so short rows cost by their
+// number what the copies, at some 60 us of latency, cost by the byte. evolve(2)
+// with periodic faces, FP64 single steps, staged / in place: 559x559x8 6.86 /
+// 11.1 ms, 353x353x20 5.26 / 6.06, 322x322x24 5.05 / 5.06, 298x298x28 4.96 /
+// 4.70, 197x197x64 4.59 / 3.63; 193x193x8 0.92 / 1.11, 158x158x12 0.83 / 0.90,
+// 136x136x16 0.776 / 0.781; 70x70x4 0.220 / 0.196.
+static bool pinned_rows(const lb_solver* s) {
+    return s->d.nz >= 24 || (int64_t)s->d.nx * s->d.ny <= 8192;
+}
+
 int lb_bind_host_fields(lb_solver* s, uint8_t* phase, double* den, double* vel, double* acc) {
     if (!s) return fail(LB_EINVAL, "null handle");
     if (s->stream) HIPCHK(hipStreamSynchronize(s->stream));
@@ -2758,8 +2769,8 @@ int lb_bind_host_fields(lb_solver* s, uint8_t* phase, double* den, double* vel, 
         HIPCHK(hipMemset(s->in_flags, 0, 4));
     }
     if (!s->h_flags && (rc = lb_host_alloc(4, (void**)&s->h_flags))) return rc;
-    s->h_pinned = pinned(phase, (size_t)ncnt) && pinned(den, (size_t)ncnt * 8) && pinned(vel, (size_t)ncnt * 24) &&
-                  pinned(acc, (size_t)ncnt * 24);
+    s->h_pinned = pinned_rows(s) && pinned(phase, (size_t)ncnt) && pinned(den, (size_t)ncnt * 8) &&
+                  pinned(vel, (size_t)ncnt * 24) && pinned(acc, (size_t)ncnt * 24);
     s->ncnt = ncnt;
     s->h_phase = phase;
     s->h_den = den;

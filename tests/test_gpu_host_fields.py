@@ -45,3 +45,10 @@ def test_pinned_fields_equal_staged_ones(lat, bc, precision, monkeypatch):
     for n, (a, b) in enumerate(zip(pinned, staged)):
         for x, y, what in zip(a, b, ("den", "vel", "f")):
             np.testing.assert_array_equal(x, y, err_msg=f"{what} after call {n}")
+
+
+@pytest.mark.parametrize("lat", [(97, 85, 23), (97, 85, 24), (128, 64, 3), (683, 12, 2)])
+def test_short_rows_equal_staged_ones(lat, monkeypatch):
+    """Both sides of the lines between staged copies and fields reached in place:
+    the length of the rows and their number."""
+    test_pinned_fields_equal_staged_ones(lat, (P, P, W, W, S, S), "fp32", monkeypatch)
