@@ -1651,20 +1651,23 @@ static bool pair_thin(const lb_solver* s) {
 }
 
 // Without timing (LB_AUTOTUNE=0): whether a lattice steps in pairs that
-// tune_pair would settle. The lines lie where pairs were never slower (ms per
-// step, single / paired). Moving lid: FP64 from 24^3 0.0078 / 0.0057 over 64^3
-// 0.0162 / 0.0160 to 256^3 0.954 / 0.628; FP32 64^3 0.0108 / 0.0123, 70^3
-// 0.0210 / 0.0139, 512x128x128 0.266 / 0.195; FP32 storage 64x64x256 0.0349 /
-// 0.0427, 100x100x100 0.0457 / 0.0407, 512x128x128 0.305 / 0.234; FP16 64^3
-// 0.0115 / 0.0134, 256^3 0.295 / 0.359. Sparse with a lid over 20% solid:
-// FP64 384x192x192 0.615 / 0.522, FP32 320^3 0.867 / 0.688. Walls at rest in
-// FP16: 64^3 0.0193 / 0.0123, 256^3 0.280 / 0.272, 320^3 0.532 / 0.532.
+// tune_pair would settle. The lines lie where pairs are not slower, with faces
+// and forces of any kind (ms per step, single in the default launch / paired).
+// Moving lid: FP64 from 24^3 0.0078 / 0.0057 over 64^3 0.0162 / 0.0160 to 256^3
+// 0.954 / 0.628; FP32 64^3 0.0108 / 0.0123, 70^3 0.0210 / 0.0139, 512x128x128
+// 0.266 / 0.195; FP32 storage 64x64x256 0.0349 / 0.0427, 100x100x100 0.0457 /
+// 0.0407, 512x128x128 0.305 / 0.234 (the one exception found: 128^3,
+// regularized, with a force field, 0.0824 / 0.0870); FP16 64^3 0.0115 / 0.0134,
+// 256^3 0.295 / 0.359. Sparse with a lid over 20% solid: FP64 384x192x192 0.615
+// / 0.522, FP32 320^3 0.867 / 0.688. Walls at rest in FP16: channel 64^3 0.0193
+// / 0.0123, 160^3 0.0951 / 0.0765; Zou-He duct 192^3 0.140 / 0.145, 256^3 0.286
+// / 0.358.
 static bool pair_untimed(const lb_solver* s) {
     switch (s->prec) {
     case LB_FP64: return true;
     case LB_FP32_SHIFTED: return s->ncell > (1 << 18);
     case LB_FP32_STORAGE: return s->ncell > (1 << 20);
-    default: return !s->moving && s->ncell <= (1 << 24);
+    default: return !s->moving && s->ncell <= (1 << 22);
     }
 }
 

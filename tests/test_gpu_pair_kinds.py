@@ -142,6 +142,7 @@ def test_single_steps_launches_on_lattices_that_pair(name, env, monkeypatch):
     ((64, 64, 256), "fp32_storage", True, False), ((65, 64, 256), "fp32_storage", True, True),
     ((24, 20, 40), "fp16", True, False), ((24, 20, 40), "fp16", False, True),
     ((24, 20, 40), "fp32", False, True), ((24, 20, 40), "fp32_storage", False, True),
+    ((256, 128, 128), "fp16", False, True), ((257, 128, 128), "fp16", False, False),
 ])
 def test_untimed_choice(lat, precision, lid, pairs, monkeypatch):
     """LB_AUTOTUNE=0 times nothing: pairs where they are never slower, single
