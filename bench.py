@@ -244,14 +244,15 @@ def headline(precs, steps, warmup, layout, solid):
 
 
 def cavity_workload(n, steps, warmup, precs):
-    """The cavity in each precision. The warm-up call is long enough (60
+    """The cavity in each precision. The warm-up call is long enough (80
     steps at least) to hold the launch tuning of a dense lattice, which times
-    up to 8 launch candidates and the pull steps on the call's own steps."""
+    up to 10 launch candidates and the pull steps on the call's own steps, and
+    after it the timing of single against paired steps."""
     import torch
     out = {}
     for prec in precs:
         s, nfl = make_cavity(n, prec)
-        t, _ = time_device(s, steps, max(warmup, 60))
+        t, _ = time_device(s, steps, max(warmup, 80))
         lay = s.engine.layout()
         pair = s.engine.paired_steps()
         gbs = bytes_per_site(prec, pair) * nfl * steps / t / 1e9

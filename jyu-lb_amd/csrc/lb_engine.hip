@@ -765,8 +765,8 @@ struct lb_solver {
     uint32_t* mov_word = nullptr;  // paired steps with moving walls: PairParams::mov, and whether it holds
     double* den2 = nullptr;        // (each site's walls share one of a few velocities); PairParams::rho_*
     bool mov_pairs = false;
-    // paired steps of the dense layouts (k_pair): the request (LB_PAIR, as
-    // sp_pull), whether run_steps takes them, and their tiling
+    // paired steps (k_pair): the request (LB_PAIR, as sp_pull), whether run_steps
+    // takes them, and their tiling
     int pair = -1;
     bool pair_on = false;
     bool pair_tune = false;  // ... to be settled by timing both (tune_pair), with single steps until then
@@ -788,7 +788,7 @@ struct lb_solver {
     uint32_t* tab = nullptr;
     uint32_t* tabc = nullptr;  // SP_CODE_BYTES per compact site: SP_WORDS rows of words, a row of bytes
     uint32_t* tabw = nullptr;
-    void* f2 = nullptr;   // sparse layout: the second population array of the pull steps (run_steps), or null
+    void* f2 = nullptr;   // the second population array of pull steps and pairs (run_steps), or null
     int sp_pull = -1;     // pull steps: 1 on, 0 off, -1 by sp_pull_on / the launch tuner (LB_SP_PULL sets 1 or 0)
     bool pull_active = false;  // run_steps takes pull steps (f2 allocated); a dense f2 may be a tuning candidate
     // the state before the last step of the last evolve call, for the
@@ -1593,19 +1593,21 @@ static void layout_defaults(lb_solver* s, int layout) {
     }
 }
 
-// Whether steps are paired (k_pair) where a call has two of them left: not with a symmetric x face (the sweep along i does not mirror), nor
-// where three planes of populations exceed the kernel's 32-bit offsets, nor
-// where LB_SP_PULL asks for single steps of one kind. rs and ps are set.
+// Whether steps are paired (k_pair) where a call has two of them left: not with
+// a symmetric x face (the sweep along i does not mirror), nor where three planes
+// of populations exceed the kernel's 32-bit offsets, nor where LB_SP_PULL asks
+// for single steps of one kind, nor on thin lattices (pair_thin), nor once steps
+// were captured (pairs_barred). rs and ps are set.
 //
 // In the sparse layout (nfluid is set) solid cells are columns that idle, every
 // first step looks its upstream sites up, and small lattices wait for that
 // chain. Measured (ms per step, single / paired): random spheres of 20% solid
-// FP64 384x192x192 0.589 / 0.483, 256x128x128 0.165 / 0.147, 320^3 1.383 /
-// 1.167, 64^3 0.0149 / 0.0150; FP32 384x192x192 0.303 / 0.289, 256x128x128
-// 0.085 / 0.088; 40% solid FP64 256^3 0.528 / 0.541. FP64 takes them; so does FP32
-// from 2^23 sites (768x384x384 2.57 / 2.28), which below lets tune_pair time
-// both; FP32 storage (320^3 0.769 / 0.831) and FP16 (0.436 /
-// 0.561) stay single.
+// FP64 384x192x192 0.592 / 0.458, 256x128x128 0.169 / 0.146, 320^3 1.389 /
+// 1.158, 64^3 0.0148 / 0.0145; FP32 384x192x192 0.320 / 0.281, 256x128x128
+// 0.087 / 0.085; 40% solid FP64 256^3 0.523 / 0.510. FP64 takes them; so does
+// FP32 from 2^23 sites (768x384x384 2.57 / 2.26), which below lets tune_pair
+// time both. FP32 storage (256x128x128 0.092 / 0.113, 384x192x192 0.328 /
+// 0.329, 320^3 0.766 / 0.725) and FP16 (320^3 0.456 / 0.618) stay single.
 static bool pair_thin(const lb_solver* s);
 static bool pair_wanted(const lb_solver* s) {
     if (s->sp_pull >= 0 || s->pair == 0 || s->captured) return false;
@@ -1838,8 +1840,8 @@ static bool give_back(lb_solver* s) {
 // Single or paired steps for the lattice and the walls as they are, or to be
 // settled by timing (tune_pair), with single steps until then. Pairs are faster
 // where walls stand still and values have 4 bytes or more (ms per step, single
-// / paired: 256^3 channel FP64 0.894 / 0.567, FP32 0.451 / 0.300; 48^3 FP64
-// 0.0215 / 0.0085). With moving walls or FP16 storage, where the collisions
+// / paired: 256^3 channel FP64 0.893 / 0.564, FP32 0.454 / 0.299; 48^3 FP64
+// 0.0215 / 0.0083). With moving walls or FP16 storage, where the collisions
 // bind, it depends (figures at pair_untimed). Sparse FP32: see pair_wanted.
 static int settle_pairs(lb_solver* s) {
     s->pair_tune = false;
@@ -2076,7 +2078,7 @@ int lb_set_face_data(lb_solver* s, int face, const double* den_face, const doubl
 // blocks of 2^12 sites): single steps FP64 384x192x192 0.666 / 0.589, 320^3
 // 1.501 / 1.383, 128x64x64 0.0261 / 0.0252, FP32 384x192x192 0.331 / 0.303,
 // 128x64x64 0.0138 / 0.0133, FP16 320^3 0.440 / 0.425; paired FP64 384x192x192
-// 0.524 / 0.497. Smaller blocks put more waves across a boundary, where the
+// 0.524 / 0.497 (in long sweeps). Smaller blocks put more waves across a boundary, where the
 // codes run out (2^10: 0.596), larger ones spread again (2^14: 0.606, 2^16:
 // 0.622). Small lattices lose by the boundaries (24x24x100 0.0063 / 0.0067).
 static uint32_t sparse_blocks(const lb_solver* s, uint64_t nfp) {

@@ -16,10 +16,11 @@
 // Only the first step of the rim is computed twice (by this tile and by its
 // neighbour), so two steps move little more than one step's bytes. Results
 // are bit-identical to single steps. Measured (ms per step, single / paired):
-// 256^3 FP64 0.894 / 0.570 (a pair moves 6.6 GB past L2, 5.8 TB/s: the rims'
-// lines, of which L2 catches about half, are what is left), FP32 0.451 /
-// 0.315 and FP16 0.274 / 0.277 (bound by the collisions' instructions);
-// 512x128x128 duct FP64 0.433 / 0.299; 32x34x8 channel 0.0185 / 0.0042.
+// 256^3 channel FP64 0.893 / 0.564 (a pair moves 5.46 GB past L2, 1.07 of its
+// populations, as L2 catches 40% of the rims: 4.8 TB/s, 0.83 of the copy),
+// FP32 0.454 / 0.299 and FP16 0.265 / 0.274 (VALU instructions issue in 75 and
+// 85% of the CUs' busy cycles; FP64 35%); 512x128x128 duct FP64 0.433 / 0.295;
+// 32x34x8 channel 0.0190 / 0.0044.
 //
 // LDS. A population with c_i = -1 is needed in the iteration it is made in,
 // one with c_i = 0 in the next, one with c_i = +1 in the one after, so the
@@ -36,7 +37,8 @@
 // four planes, each loaded an iteration ahead. Tiles' rows start and end
 // anywhere in a line: L2 joins the stores (1.80 GB written for 1.72 GB of
 // populations on 384x192x192 cells of 20% solid). ms per step there, single /
-// paired: FP64 0.589 / 0.483; 256x128x128 0.165 / 0.147.
+// paired: FP64 0.592 / 0.458; 256x128x128 0.169 / 0.146. The indices take the
+// 16 KiB of LDS that FP64's rings leave of 160.
 #pragma once
 #include <type_traits>
 
@@ -94,13 +96,15 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
     constexpr int NT = pair_threads(P), NC = pair_cells(P);
     // The gather's loads that are issued before the first step; the others
     // follow it, and have the second step's time to arrive. Measured (ms per
-    // step, all 19 first / 14): FP32 256^3 0.322 / 0.300, sparse 256x128x128
-    // 0.103 / 0.090; sparse FP64 384x192x192 0.501 / 0.492; but dense FP64
-    // 256^3, which waits for memory as it is, 0.566 / 0.595.
+    // step, all 19 first / 14): FP32 256^3 0.322 / 0.300; dense FP64 256^3,
+    // which waits for memory as it is, 0.566 / 0.595; with the sparse sweeps as
+    // long as the dense ones, FP32 256x128x128 0.103 / 0.090 and FP64
+    // 384x192x192 0.501 / 0.492.
     constexpr int FIRST = (P == LB_FP64 && !SP) || (MOV && FULL) ? Q : 14;
     auto in_part = [](int part, int l) constexpr { return part < 0 || (l < FIRST) == (part == 0); };
     __shared__ TS ring[RING_SLOTS * NT];
     __shared__ uint32_t idx[SP ? 4 * NC : 1];
+    static_assert(sizeof(ring) + (SP ? sizeof(idx) : 0) <= 160 * 1024, "a CU has 160 KiB of LDS");
 
     // tile and chunk of this workgroup: each XCD takes a contiguous range, so
     // that neighbouring tiles, which read each other's rims, share its L2
@@ -462,8 +466,9 @@ __global__ __launch_bounds__(pair_threads(P)) void k_pair(StepParams p, PairPara
         asm volatile("" : "+v"(mNN));
         if (second) {
             // Plain stores: L2 joins the lines that two tiles share. With
-            // non-temporal ones 256^3 FP64 ran 0.615 ms per step (plain
-            // 0.572) and tiles that split lines 0.968 (33x12x32; 0.751).
+            // non-temporal ones 256^3 FP64 ran 0.615 ms per step (plain 0.572
+            // in the same session) and tiles that split lines 0.968 (33x12x32;
+            // 0.751).
             uint64_t step = (uint64_t)psb;
             if constexpr (SP) {
                 uint64_t a = (uint64_t)((TS*)p.f2 + nB);
