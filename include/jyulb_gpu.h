@@ -298,10 +298,11 @@ int lb_pull_steps(lb_solver *s, int *on);
 
 /* Whether lb_evolve takes two steps per pass over the populations (no
  * counterpart in the reference) where a call has two left: into a second
- * population array, allocated by the first such call; without the memory for
- * it steps stay single. Where it depends on the flow, the first call that is
- * long enough times both, and *on is 0 until then. LB_PAIR=0/1 in the
- * environment decides instead. Results are identical either way. */
+ * population array, allocated by the first such call; without room for it
+ * (lb_pair_bytes) steps stay single. Where it depends on the flow, the first
+ * call with more than 21 steps times both, from 2^22 cells on after the launch
+ * tuning's 10 to 51, and *on is 0 until then. LB_PAIR=0/1 in the environment
+ * decides instead. Results are identical either way. */
 int lb_paired_steps(lb_solver *s, int *on);
 
 /* Device memory that the handle holds for paired steps only: the second
