@@ -1593,6 +1593,8 @@ static void layout_defaults(lb_solver* s, int layout) {
     }
 }
 
+static bool pair_thin(const lb_solver* s);
+
 // Whether steps are paired (k_pair) where a call has two of them left: not with
 // a symmetric x face (the sweep along i does not mirror), nor where three planes
 // of populations exceed the kernel's 32-bit offsets, nor where LB_SP_PULL asks
@@ -1608,7 +1610,6 @@ static void layout_defaults(lb_solver* s, int layout) {
 // FP32 from 2^23 sites (768x384x384 2.57 / 2.26), which below lets tune_pair
 // time both. FP32 storage (256x128x128 0.092 / 0.113, 384x192x192 0.328 /
 // 0.329, 320^3 0.766 / 0.725) and FP16 (320^3 0.456 / 0.618) stay single.
-static bool pair_thin(const lb_solver* s);
 static bool pair_wanted(const lb_solver* s) {
     if (s->sp_pull >= 0 || s->pair == 0 || s->captured) return false;
     if (s->d.bc[0] == SYMMETRIC || s->d.bc[1] == SYMMETRIC) return false;
@@ -2327,6 +2328,18 @@ static void one_step(lb_solver* s, StepParams& p, int& odd) {
     }
 }
 
+// Whether the stream is being captured (or does not say): nothing may be timed
+// or waited for then. Remembers that steps were captured.
+static bool capturing(lb_solver* s) {
+    hipStreamCaptureStatus now = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s->stream, &now) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    if (now != hipStreamCaptureStatusNone) s->captured = true;
+    return now != hipStreamCaptureStatusNone;
+}
+
 // Whether this call's steps have to stay single. A captured graph replays with
 // the arrays that its steps were captured with, while a pair leaves the state
 // in the other array: a pair between two replays would have the next replay
@@ -2334,16 +2347,8 @@ static void one_step(lb_solver* s, StepParams& p, int& odd) {
 // this handle's later ones, in the array that the graph holds; the second
 // array goes back at the first call outside a capture.
 static bool pairs_barred(lb_solver* s) {
-    hipStreamCaptureStatus now = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s->stream, &now) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;  // this call only
-    }
-    if (now != hipStreamCaptureStatusNone) {
-        s->captured = true;
-    } else if (s->captured && (s->pair_on || s->pair_tune)) {
-        drop_pairs(s);
-    }
+    if (capturing(s)) return true;
+    if (s->captured && (s->pair_on || s->pair_tune)) drop_pairs(s);
     return s->captured;
 }
 
@@ -2661,10 +2666,10 @@ static int capture_prev(lb_solver* s) {
 // first long call, then the steps (den/vel stored on the last one).
 static int evolve_steps(lb_solver* s, uint32_t steps) {
     int rc = LB_OK;
-    const bool barred = pairs_barred(s);
+    const bool now = capturing(s), barred = pairs_barred(s);
     if (s->prec == LB_FP16_STORAGE && (s->f16_dirty || s->f16_since >= s->f16_check) && (rc = fp16_guard(s)))
         return rc;
-    if (s->tune && !pairs_used(s)) {
+    if (s->tune && !now && !pairs_used(s)) {
         // tuning takes TUNE_WARM + TUNE_STEPS per candidate of this call's
         // steps; a shorter call leaves it to a later one
         StepCfg c[TUNE_MAX];

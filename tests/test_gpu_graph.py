@@ -60,3 +60,29 @@ def test_replays_between_plain_calls(lat, bc, precision, layout, solid, lid, bef
                                   (ref.download_post_f(), *ref.download_den_vel()), ("f", "den", "vel")):
                 np.testing.assert_array_equal(a, b, err_msg=f"{what} after replay {n}")
     assert not e.paired_steps()
+
+
+@pytest.mark.parametrize("layout,lid", [("rows", False), ("rows", True), ("sparse", False)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_a_captured_call_times_nothing(precision, layout, lid, monkeypatch):
+    """A call long enough for the launch tuner and for the timing of pairs,
+    captured; then plain ones, which may tune."""
+    import torch
+    monkeypatch.setenv("LB_AUTOTUNE_MIN_CELLS", "0")
+    st = torch.cuda.Stream()
+    e, ref = (_engine((20, 16, 30), (W,) * 6, precision, layout, 0.1 if layout == "sparse" else 0.0, lid, st)
+              for _ in range(2))
+    print(f"{precision} {layout} lid {lid}", flush=True)
+    with torch.cuda.stream(st):
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        g.capture_begin()
+        e.evolve(80)
+        g.capture_end()
+        for n, plain in enumerate((80, 2, 100)):
+            g.replay()
+            torch.cuda.synchronize()
+            ref.evolve(80)
+            e.evolve(plain)
+            ref.evolve(plain)
+            np.testing.assert_array_equal(e.download_post_f(), ref.download_post_f(), err_msg=f"after replay {n}")
